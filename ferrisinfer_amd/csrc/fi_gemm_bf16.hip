@@ -13,8 +13,8 @@
 // which is the B operand of one 16x16x32 MFMA per (slab, step) for lane `lane`: every wave
 // load is 16 contiguous bytes per lane and one group's K step is 16 KiB contiguous.
 //
-// Kernel: a workgroup of 4 waves computes a (16 MT) x (64 NT) tile over one split's K range
-// (MT = 8, 6 or 4 row tiles above 64 rows, chosen per shape so the busiest CU gets the least
+// Kernel (above 64 rows, and the greedy head): a workgroup of 4 waves computes a (16 MT) x (64 NT)
+// tile over one split's K range (MT = 8, 6 or 4 row tiles above 64 rows, chosen per shape so the busiest CU gets the least
 // work).  The activation block (16 MT rows x 32 k, or 64 k for bf16 activations) is staged per
 // step through double-buffered LDS: f32 activations are rounded to bf16 (nearest even) on the
 // way in, bf16 activations (rounded the same way by their producer) are copied, so both give
@@ -26,6 +26,7 @@
 // fastest, then column group, then split): the row blocks that share a column group's weights
 // run together on one L2.
 #include <algorithm>
+#include <type_traits>
 
 #include "fi_common.h"
 #include "fi_device.h"
@@ -337,9 +338,234 @@ __global__ __launch_bounds__(kThreads, kOccupancy) void gemm_bf16_kernel(BGemmAr
   store_tile<MT, NT, EPI>(g, acc, m0, slab0, z, lane);
 }
 
+// ---- few rows: the weight stream is the work ----
+// Up to 64 rows a product reads each weight byte for at most 64 multiply-adds, so the HBM stream
+// bounds it.  A workgroup of SW x KW waves owns SW * NS slabs and one split's K range, cut into
+// KW consecutive parts: wave (sw, kw) streams its NS slabs' fragments of part kw into a register
+// ring DEPTH steps deep.  The activations of DEPTH steps of every part are one stage: loaded to
+// registers at the start of the stage before (ahead of that stage's weight loads, which return
+// after them and so stay in flight at its end), then put in LDS in fragment order, where the SW
+// waves of the part share them.  The KW partial sums meet in LDS and are added in part order, so
+// a consumer reads a few partials instead of up to 32, and SwiGLU needs none.
+// Llama-3-8B's MLP, weights from HBM, against the kernel above: 16 rows, w1|w3 51 + 4.8 (its split
+// sum) -> 42.5 us (5.5 TB/s), w2 24 -> 22 us (5.3 TB/s); 64 rows, 69.7 + 9.4 -> 51 us and
+// 32.5 -> 29.3 us.  What is left over a plain stream grows with the rows: each workgroup reads
+// the activations of its K range from L2.
+template <int MT, int NS, int SW, int KW, int DEPTH, int EPI, bool KTAIL, bool A16>
+__global__ __launch_bounds__(64 * SW * KW, 2) void gemm_bf16_rows_kernel(BGemmArgs g) {
+  constexpr int AV = A16 ? 1 : 2;              // 16-byte loads of an activation fragment and lane
+  constexpr int FRAGS = DEPTH * MT;            // 1 KiB bf16 fragments of a part's stage
+  constexpr int A_PER = (FRAGS + SW - 1) / SW; // per wave
+  constexpr int A_BYTES = 2 * KW * FRAGS * 1024, P_BYTES = KW * SW * MT * NS * 1024;
+  __shared__ __align__(16) unsigned char s_mem[A_BYTES > P_BYTES ? A_BYTES : P_BYTES];
+  uint4* const s_a = reinterpret_cast<uint4*>(s_mem);  // [2][KW][DEPTH][MT][64]
+  // wave indices in scalar registers: the step counts that depend on them guard MFMAs, which a
+  // lane mask would not
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int sw = w % SW, kw = w / SW;
+  const int li = lane & 15, lk = lane >> 4;
+  const int slab0 = (static_cast<int>(blockIdx.x) * SW + sw) * NS, z = static_cast<int>(blockIdx.y);
+  const int q0 = z * g.q_per_split;
+  const int nq = min(g.q_per_split, g.q_total - q0);
+  const int per = (nq + KW - 1) / KW;          // steps of a part; the last ones may hold fewer or none
+  const int s0 = min(kw * per, nq);
+  const int n = min(per, nq - s0);
+  const int nst = (per + DEPTH - 1) / DEPTH;   // stages, the same for every wave
+
+  const uint4* bbase = reinterpret_cast<const uint4*>(g.bp) +
+                       ((size_t)(slab0 / kGroupSlabs) * g.q_total * kGroupSlabs + slab0 % kGroupSlabs) * 64 + lane;
+  uint4 ring[DEPTH][NS];
+  // past the part's end a step of the split is read again and not used
+  auto step_at = [&](int step) { return q0 + min(s0 + max(min(step, n - 1), 0), nq - 1); };
+  auto issue = [&](int step, uint4 (&ws)[NS]) {
+    const int q = step_at(step);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) ws[s] = bbase[((size_t)q * kGroupSlabs + s) * 64];
+  };
+  uint4 areg[A_PER][AV];
+  int ak[A_PER];  // KTAIL: K index of the lane's first element
+  auto load_a = [&](int stage) {
+#pragma unroll
+    for (int r = 0; r < A_PER; ++r) {
+      const int f = min(sw + r * SW, FRAGS - 1);
+      const int kk = step_at(stage * DEPTH + f / MT) * kStepK + 8 * lk;
+      const int row = min(16 * (f % MT) + li, g.m - 1);
+      if constexpr (KTAIL) ak[r] = kk;
+      if constexpr (A16) {
+        const uint16_t* a = static_cast<const uint16_t*>(g.a) + (size_t)row * g.lda;
+        areg[r][0] = *reinterpret_cast<const uint4*>(a + (KTAIL ? min(kk, ((g.k + 7) & ~7) - 8) : kk));
+      } else {
+        const float* a = static_cast<const float*>(g.a) + (size_t)row * g.lda;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          areg[r][h] = *reinterpret_cast<const uint4*>(a + (KTAIL ? min(kk + 4 * h, ((g.k + 3) & ~3) - 4) : kk + 4 * h));
+      }
+    }
+  };
+  auto store_a = [&](int buf) {
+#pragma unroll
+    for (int r = 0; r < A_PER; ++r) {
+      if (FRAGS % SW != 0 && sw + r * SW >= FRAGS) continue;
+      uint4 x = areg[r][0];
+      if constexpr (!A16) {
+        const float4 lo = __builtin_bit_cast(float4, areg[r][0]), hi = __builtin_bit_cast(float4, areg[r][1]);
+        const uint2 a = __builtin_bit_cast(uint2, __builtin_convertvector((f32x4{lo.x, lo.y, lo.z, lo.w}), bf16x4));
+        const uint2 b = __builtin_bit_cast(uint2, __builtin_convertvector((f32x4{hi.x, hi.y, hi.z, hi.w}), bf16x4));
+        x = make_uint4(a.x, a.y, b.x, b.y);
+      }
+      if constexpr (KTAIL) {
+        // elements past K read as zero (a clamped load starts at or before K's last elements)
+        uint32_t xw[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t lo = ak[r] + 2 * e < g.k ? (xw[e] & 0xffffu) : 0u;
+          const uint32_t hi = ak[r] + 2 * e + 1 < g.k ? (xw[e] & 0xffff0000u) : 0u;
+          xw[e] = lo | hi;
+        }
+        x = make_uint4(xw[0], xw[1], xw[2], xw[3]);
+      }
+      s_a[((buf * KW + kw) * FRAGS + sw + r * SW) * 64 + lane] = x;
+    }
+  };
+  v4f acc[MT][NS];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int s = 0; s < NS; ++s) acc[t][s] = v4f{0.f, 0.f, 0.f, 0.f};
+
+  load_a(0);
+  sched_fence();
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) issue(d, ring[d]);
+  store_a(0);
+  __syncthreads();
+  auto stage = [&](int st, auto more) {
+    sched_fence();
+    if constexpr (decltype(more)::value) {
+      load_a(st + 1);
+      sched_fence();
+    }
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      const int step = st * DEPTH + d;
+      if (step < n) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          const bf16x8 af =
+              __builtin_bit_cast(bf16x8, s_a[(((st & 1) * KW + kw) * FRAGS + d * MT + t) * 64 + lane]);
+#pragma unroll
+          for (int s = 0; s < NS; ++s)
+            acc[t][s] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, __builtin_bit_cast(bf16x8, ring[d][s]), acc[t][s], 0, 0, 0);
+        }
+      }
+      if constexpr (decltype(more)::value) issue(step + DEPTH, ring[d]);
+      sched_fence();
+    }
+    if constexpr (decltype(more)::value) store_a((st & 1) ^ 1);
+    __syncthreads();
+  };
+  for (int st = 0; st + 1 < nst; ++st) stage(st, std::true_type{});
+  stage(nst - 1, std::false_type{});
+  if constexpr (KW == 1) {
+    store_tile<MT, NS, EPI>(g, acc, 0, slab0, z, lane);
+    return;
+  } else {
+    v4f* const s_part = reinterpret_cast<v4f*>(s_mem);  // [KW][SW][MT * NS][64]
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int s = 0; s < NS; ++s) s_part[((kw * SW + sw) * MT * NS + t * NS + s) * 64 + lane] = acc[t][s];
+    __syncthreads();
+    // wave (sw, kw) adds and stores row tiles kw, kw + KW, ... of its slabs
+#pragma unroll
+    for (int t0 = 0; t0 < MT; t0 += KW) {
+      const int t = t0 + kw;
+      if (t >= MT) return;
+      v4f sum[1][NS];
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        sum[0][s] = s_part[(sw * MT * NS + t * NS + s) * 64 + lane];
+#pragma unroll
+        for (int src = 1; src < KW; ++src) sum[0][s] += s_part[((src * SW + sw) * MT * NS + t * NS + s) * 64 + lane];
+      }
+      store_tile<1, NS, EPI>(g, sum, 16 * t, slab0, z, lane);
+    }
+  }
+}
+
 int32_t q_steps(int32_t k) { return (k + kStepK - 1) / kStepK; }
 
 constexpr int kNt = 4;  // slabs per wave: a workgroup covers 256 columns
+
+constexpr int kRowsMax = 64;   // gemm_bf16_rows_kernel up to this many rows
+constexpr int kRowsStage = 8;  // K steps per stage (4 where two stages would pass 128 KiB of LDS)
+constexpr int kRowsParts = 2;  // K parts of a workgroup of the split-K products
+
+template <int MT, int NS, int SW, int KW, int EPI, bool A16>
+void launch_rows_as(fi_context* ctx, const BGemmArgs& g) {
+  constexpr int DEPTH = 2 * KW * MT * kRowsStage <= 128 ? kRowsStage : 4;
+  const dim3 grid(static_cast<unsigned>((g.slabs + SW * NS - 1) / (SW * NS)), static_cast<unsigned>(g.splits));
+  if (g.k % kStepK == 0) {
+    hipLaunchKernelGGL((gemm_bf16_rows_kernel<MT, NS, SW, KW, DEPTH, EPI, false, A16>), grid, dim3(64 * SW * KW), 0,
+                       ctx->stream, g);
+  } else {
+    hipLaunchKernelGGL((gemm_bf16_rows_kernel<MT, NS, SW, KW, DEPTH, EPI, true, A16>), grid, dim3(64 * SW * KW), 0,
+                       ctx->stream, g);
+  }
+}
+
+// Slabs a workgroup of the split-K products owns: eight (4 x 2 waves of two slabs), or four where
+// that would leave fewer than 32 workgroups a split (56 slabs, K 4864, 64 rows: 6.1 us against
+// 8.9 us of the kernel above).
+int rows_slabs(int slabs) { return slabs >= 256 ? 8 : 4; }
+
+template <int MT, int EPI, bool A16>
+void launch_rows_mt(fi_context* ctx, const BGemmArgs& g) {
+  if constexpr (EPI == kEpiSwiglu) {
+    // one launch without partials; a workgroup takes eight slabs where that still gives 128 of
+    // them (1792 slabs: 42.5 us against 54 us with four slabs and K in four parts), else four
+    // (608 slabs, 64 rows: 9.2 us against 13.2 us with eight)
+    if (g.slabs >= 1024)
+      launch_rows_as<MT, 2, 4, 2, EPI, A16>(ctx, g);
+    else
+      launch_rows_as<MT, 2, 2, 4, EPI, A16>(ctx, g);
+  } else if (rows_slabs(g.slabs) == 4) {
+    launch_rows_as<MT, 1, 4, kRowsParts, EPI, A16>(ctx, g);
+  } else {
+    launch_rows_as<MT, 2, 4, kRowsParts, EPI, A16>(ctx, g);
+  }
+}
+
+template <int EPI>
+int32_t launch_rows(fi_context* ctx, const BGemmArgs& g, bool a16) {
+  const int mt = g.m > 32 ? 4 : (g.m > 16 ? 2 : 1);
+  if (mt == 4)
+    a16 ? launch_rows_mt<4, EPI, true>(ctx, g) : launch_rows_mt<4, EPI, false>(ctx, g);
+  else if (mt == 2)
+    a16 ? launch_rows_mt<2, EPI, true>(ctx, g) : launch_rows_mt<2, EPI, false>(ctx, g);
+  else
+    a16 ? launch_rows_mt<1, EPI, true>(ctx, g) : launch_rows_mt<1, EPI, false>(ctx, g);
+  FI_CHECK_LAUNCH("gemm_bf16_rows_kernel");
+  return FI_OK;
+}
+
+// Splits of a product of few rows: about one workgroup per CU, every split a whole number of
+// stages where K allows (a part of 11 steps runs as long as one of 16).  Two workgroups per CU
+// measured no better (16 rows, K 14336, 256 slabs: 23.2 against 22.1 us) and their consumer reads
+// twice the partials.
+int rows_splits(fi_context* ctx, int q, int slabs) {
+  const int cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
+  const int groups = (slabs + rows_slabs(slabs) - 1) / rows_slabs(slabs);
+  const int unit = kRowsStage * kRowsParts;
+  const int stages = (q + unit - 1) / unit;
+  const int want = std::max(1, (cus + groups / 2) / groups);
+  const int each = std::max(1, (stages + want / 2) / want);  // stages per split
+  const int per = std::min(q, unit * each);
+  const int s = (q + per - 1) / per;
+  const int even = (q + s - 1) / s;
+  return (q + even - 1) / even;  // every split non-empty
+}
 
 #ifndef FI_BGEMM_FORCE_MT
 #define FI_BGEMM_FORCE_MT 0  // a fixed row tile count above 64 rows (0: chosen per shape)
@@ -376,6 +602,7 @@ int mt_for(fi_context* ctx, int m, int slabs) {
 // kernel's ~40 % of the bf16 peak per CU), plus each extra partial written and read back at
 // ~6 TB/s (wo at M 2304: 2 splits, 100 -> 83 us with the consumer 23 -> 31 us).
 int split_count(fi_context* ctx, int m, int k, int slabs) {
+  if (m <= kRowsMax) return rows_splits(ctx, q_steps(k), slabs);
   const int mt = mt_for(ctx, m, slabs);
   const int mblocks = (m + 16 * mt - 1) / (16 * mt);
   const int groups = (slabs + kWaves * kNt - 1) / (kWaves * kNt);
@@ -428,6 +655,14 @@ void launch_mt(fi_context* ctx, const BGemmArgs& g, bool a16) {
 
 template <int EPI>
 int32_t launch_bgemm(fi_context* ctx, BGemmArgs g, int splits, bool a16) {
+  // the head's single K range and its per-tile states suit the kernel above at every row count
+  // (5 rows x 128256 columns: 182 us against 202 us)
+  if constexpr (EPI == kEpiPartial || EPI == kEpiSwiglu) {
+    if (g.m <= kRowsMax) {
+      g.splits = splits;
+      return launch_rows<EPI>(ctx, g, a16);
+    }
+  }
   const int mt = mt_for(ctx, g.m, g.slabs);
   g.mblocks = (g.m + 16 * mt - 1) / (16 * mt);
   g.groups = (g.slabs + kWaves * kNt - 1) / (kWaves * kNt);
@@ -443,11 +678,13 @@ int32_t launch_bgemm(fi_context* ctx, BGemmArgs g, int splits, bool a16) {
     case 4:
       launch_mt<4, EPI>(ctx, g, a16);
       break;
-    case 2:
-      launch_mt<2, EPI>(ctx, g, a16);
-      break;
-    default:
-      launch_mt<1, EPI>(ctx, g, a16);
+    default:  // 64 rows or fewer: only the greedy head comes here
+      if constexpr (EPI == kEpiArgmax) {
+        if (mt == 2)
+          launch_mt<2, EPI>(ctx, g, a16);
+        else
+          launch_mt<1, EPI>(ctx, g, a16);
+      }
       break;
   }
   FI_CHECK_LAUNCH("gemm_bf16_kernel");
@@ -649,7 +886,7 @@ int32_t fi_gemm_bf16_swiglu(fi_context* ctx, const void* d_a, int32_t a_dtype, i
   g.lda = lda;
   g.q_total = q_steps(k);
   g.slabs = data_slabs(n, true);
-  const int splits = split_count(ctx, m, k, g.slabs);
+  const int splits = m <= kRowsMax ? 1 : split_count(ctx, m, k, g.slabs);
   if (splits == 1) {  // the epilogue applies SwiGLU directly
     g.out = static_cast<float*>(d_out);
     g.out_bf16 = out_dtype == FI_DTYPE_BF16;

@@ -313,3 +313,57 @@ def test_convert_f32_to_bf16(orc, gpu_ctx, n, offset):
     assert np.array_equal(got[:n][~nan], want[~nan])
     assert np.all((got[:n][nan] & 0x7f80) == 0x7f80) and np.all((got[:n][nan] & 0x7f) != 0)
     assert got[n] == 0x1234  # nothing written past n
+
+
+@pytest.mark.parametrize("m", [1, 16, 17, 32, 33, 64, 65])
+@pytest.mark.parametrize("k,n", [(24, 4090), (1000, 4112), (4864, 896), (520, 8200)])
+def test_bf16_few_rows_edges(gpu_ctx, m, k, n):
+    """Both sides of every row-tile and slab-count choice up to 64 rows (and the first row count
+    past it), K shorter than one step, with a tail, an uneven last part and several stages:
+    partials and SwiGLU against f64 on the same bf16 operands.  Products are exact in f32, so
+    only the f32 sums differ: 1e-5 normwise; f32 and bf16 activations agree bit for bit."""
+    import torch
+
+    print(f"bf16 few rows m={m} k={k} n={n}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m + k + n)
+    normal = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    a16 = torch.full((m, (k + 7) // 8 * 8), float("nan"), device="cuda", dtype=torch.bfloat16)
+    a16[:, :k] = normal(m, k)
+    a32 = a16.float()
+    w, w3 = (normal(k, n) * 0.02).bfloat16(), (normal(k, n) * 0.02).bfloat16()
+    exact = a16[:, :k].double() @ w.double()
+    bp, pair = gpu_ctx.weight_pack_bf16(w, k, n), gpu_ctx.weight_pack_bf16_pair(w, w3, k, n)
+
+    def err(got, want):
+        return ((got.double() - want).norm() / want.norm()).item()
+
+    for splits in sorted({1, gpu_ctx.gemm_bf16_splits(m, k, n)}):
+        parts = [torch.full((splits, m, n), float("nan"), device="cuda") for _ in range(2)]
+        for a, out in zip((a16, a32), parts):
+            gpu_ctx.gemm_bf16(a[:, :k], bp, k, n, splits, out)
+        assert torch.equal(parts[0], parts[1])
+        assert err(parts[0].sum(dim=0), exact) <= 1e-5, splits
+    act = [torch.full((m, n), float("nan"), device="cuda") for _ in range(2)]
+    for a, out in zip((a16, a32), act):
+        gpu_ctx.gemm_bf16_swiglu(a[:, :k], pair, k, n, out)
+    assert torch.equal(act[0], act[1])
+    assert err(act[0], exact * torch.nn.functional.silu(a16[:, :k].double() @ w3.double())) <= 1e-5
+
+
+@pytest.mark.parametrize("rows", [1, 256, 257])
+def test_residual_norm_wide_rows(gpu_ctx, rows):
+    """Rows of 2048 columns and more, on both sides of the row count that takes wide workgroups,
+    against f64; 4101 columns take the scalar loop."""
+    import torch
+
+    for hidden in (2048, 4096, 4101, 33000):
+        print(f"wide residual norm rows={rows} hidden={hidden}", flush=True)
+        g = torch.Generator(device="cuda").manual_seed(rows + hidden)
+        normal = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+        parts, res, w = normal(3, rows, hidden), normal(rows, hidden), normal(hidden)
+        total, out = torch.empty_like(res), torch.empty_like(res)
+        gpu_ctx.splitk_residual_rms_norm(parts, 3, None, res, total, w, out, 1e-6)
+        want = parts.double().sum(dim=0) + res.double()
+        normed = want / (want.square().mean(dim=1, keepdim=True) + 1e-6).sqrt() * w.double()
+        for got, exact in ((total, want), (out, normed)):
+            assert ((got.double() - exact).norm() / exact.norm()).item() <= 1e-6

@@ -7,6 +7,7 @@
 // (block, kv_head) is a contiguous block_size*D run: a 16-token f32 block of D=128 is 8 KiB
 // read with 16-byte loads.
 #include <mutex>
+#include <type_traits>
 
 #include "fi_common.h"
 #include "fi_device.h"
@@ -109,11 +110,38 @@ struct DecodeArgs {
   int parts_per_seq;
   int hq;
   int hkv;
-  int group;
+  int group;       // query heads per kv head
+  int heads_per;   // of them, the heads of one workgroup (gridDim.y workgroups share the group)
   int block_size;
   int num_blocks;
   float scale;
 };
+
+// The query heads of one workgroup: `pair` numbers (sequence, kv head), `share` the part of its
+// group (gridDim.y shares, so that a pair's workgroups lie gridDim.x apart: where that is a
+// multiple of 8 they run on one XCD and its L2 serves the second read of their K/V).
+struct HeadUnit {
+  int seq, kvh;
+  int first;     // first query head of the share, within the sequence
+  int heads;     // <= 0: the group has no heads left for this share
+  size_t head0;  // first query head of the share over the batch
+};
+
+template <bool SHARES>
+__device__ __forceinline__ HeadUnit head_unit(const DecodeArgs& a, int pair) {
+  HeadUnit u;
+  u.seq = pair / a.hkv;
+  u.kvh = pair - u.seq * a.hkv;
+  u.first = u.kvh * a.group;
+  u.heads = a.group;
+  if constexpr (SHARES) {
+    const int skip = static_cast<int>(blockIdx.y) * a.heads_per;
+    u.first += skip;
+    u.heads = min(a.heads_per, a.group - skip);
+  }
+  u.head0 = (size_t)u.seq * a.hq + u.first;
+  return u;
+}
 
 // Orders this wave's LDS stores before its later LDS loads by other lanes (a compiler
 // barrier only: a wave's LDS operations execute in order).
@@ -137,11 +165,10 @@ __device__ __forceinline__ float load_partial(float* p) {
 // same arithmetic, in the same order, runs in decode_merge_kernel and in the partition
 // kernel's last-arriving workgroup, so both give identical outputs.
 template <int D, int MAXG, bool COHERENT>
-__device__ __forceinline__ void merge_unit(const DecodeArgs& a, size_t head0, int nparts, float (*s_w)[kMaxParts],
-                                           float* s_inv) {
+__device__ __forceinline__ void merge_unit(const DecodeArgs& a, size_t head0, int group, int nparts,
+                                           float (*s_w)[kMaxParts], float* s_inv) {
   constexpr int kPrefetch = 8;
   constexpr int kPerThread = (MAXG * D + kThreads - 1) / kThreads;
-  const int group = a.group;
   const int tid = threadIdx.x;
   const int w = tid >> 6;
   const int lane = tid & 63;
@@ -206,12 +233,13 @@ __device__ __forceinline__ void merge_unit(const DecodeArgs& a, size_t head0, in
 // is qkv_rope_append4_kernel's (fi::qkv_value4, fi::rope4, fi::put_kv4), so the rows equal
 // that kernel's bit for bit.
 template <int D, typename KVT, int G>
-__device__ __forceinline__ void qkv_prologue(const DecodeArgs& a, int seq, int kvh, bool append, float (*s_q)[D],
+__device__ __forceinline__ void qkv_prologue(const DecodeArgs& a, const HeadUnit& u, bool append, float (*s_q)[D],
                                              int tid, int ctx_raw) {
+  const int seq = u.seq, kvh = u.kvh;
   const int half = a.rotary_dims / 2;
   const int pass = D - 2 * half;
   const int qph = (half + pass) / 4;  // four-column items per head row
-  const int group = a.group;
+  const int group = u.heads;
   const int qw = a.hq * D, kw = a.hkv * D;
   const int width = qw + 2 * kw;
   const size_t plane = (size_t)a.num_seqs * width;
@@ -231,8 +259,8 @@ __device__ __forceinline__ void qkv_prologue(const DecodeArgs& a, int seq, int k
     if (idx < rot_items) {
       const int g = idx / qph, r = 4 * (idx - g * qph);
       const bool is_q = g < group;
-      const int col0 = is_q ? (kvh * group + g) * D : qw + kvh * D;
-      const int bcol0 = is_q ? (kvh * group + g) * D : kvh * D;
+      const int col0 = is_q ? (u.first + g) * D : qw + kvh * D;
+      const int bcol0 = is_q ? (u.first + g) * D : kvh * D;
       const float* bias = is_q ? a.bias_q : a.bias_k;
       if (r < half) {
         // a decode token's position is its sequence's last key, context_lens - 1: the table
@@ -278,7 +306,8 @@ __device__ __forceinline__ void qkv_prologue(const DecodeArgs& a, int seq, int k
   }
 }
 
-// One workgroup = one (sequence, kv_head, partition of 4*WT tokens); partitions are
+// One workgroup = one (sequence, kv_head, partition of 4*WT tokens), or in small launches a share
+// of its query heads (head_split); partitions are
 // numbered fastest across (sequence, kv_head) so the first-dispatched workgroups hold the
 // full leading partitions and the ragged tails come last.  The GQA group of query heads
 // sharing the kv head is processed together so every K/V byte is read once.
@@ -299,7 +328,7 @@ __device__ __forceinline__ void qkv_prologue(const DecodeArgs& a, int seq, int k
 // otherwise each workgroup stores (max, sum, unnormalised acc), and the last workgroup of the
 // (sequence, kv_head) group to finish merges them (counters given), or decode_merge_kernel
 // does in a launch of its own.
-template <int D, typename KVT, int G, int WT>
+template <int D, typename KVT, int G, int WT, bool SHARES>
 __global__ __launch_bounds__(kThreads) void decode_partition_kernel(DecodeArgs a) {
   constexpr int kWaveTokens = WT;
   constexpr int kPartTokens = kWaves * WT;
@@ -333,12 +362,12 @@ __global__ __launch_bounds__(kThreads) void decode_partition_kernel(DecodeArgs a
 
   const KVT* __restrict__ k_cache = static_cast<const KVT*>(a.k_cache);
   const KVT* __restrict__ v_cache = static_cast<const KVT*>(a.v_cache);
-  const int group = a.group;
-  const int units = a.num_seqs * a.hkv;
-  const int part = blockIdx.x / units;
-  const int unit = blockIdx.x - part * units;
-  const int seq = unit / a.hkv;
-  const int kvh = unit - seq * a.hkv;
+  const int pairs = a.num_seqs * a.hkv;
+  const int part = blockIdx.x / pairs;
+  const int pair = blockIdx.x - part * pairs;
+  const HeadUnit hu = head_unit<SHARES>(a, pair);
+  const int seq = hu.seq, kvh = hu.kvh, group = hu.heads;
+  if (SHARES && group <= 0) return;  // every partition of the share
   const int tid = threadIdx.x;
   int ctx = a.context_lens[seq];
   const int ctx_raw = ctx;
@@ -346,12 +375,12 @@ __global__ __launch_bounds__(kThreads) void decode_partition_kernel(DecodeArgs a
     if (part == 0 && tid == 0) atomicOr(a.faults, FI_FAULT_CONTEXT_RANGE);
     ctx = a.parts_per_seq * kPartTokens;
   }
-  const size_t head0 = (size_t)seq * a.hq + (size_t)kvh * group;  // first query head of the group
+  const size_t head0 = hu.head0;
   const bool fused = a.qkv_parts != nullptr;  // uniform
   if (ctx <= 0) {  // no keys: defined output of zeros (the new token's K/V still appended)
     if (part == 0) {
       for (int i = tid; i < group * D; i += kThreads) a.out[head0 * D + i] = 0.0f;
-      if (fused) qkv_prologue<D, KVT, G>(a, seq, kvh, true, s_q, tid, ctx_raw);
+      if (fused) qkv_prologue<D, KVT, G>(a, hu, true, s_q, tid, ctx_raw);
     }
     return;
   }
@@ -406,8 +435,9 @@ __global__ __launch_bounds__(kThreads) void decode_partition_kernel(DecodeArgs a
     ids[i] = lb < a.max_blocks ? a.block_tables[(size_t)seq * a.max_blocks + lb] : -1;
   }
   if (fused) {
-    // the last partition holds the new token: its K/V row is written before the keys are read
-    qkv_prologue<D, KVT, G>(a, seq, kvh, part == nparts - 1, s_q, tid, ctx_raw);
+    // the last partition holds the new token: its K/V row is written before the keys are read (by
+    // every share's workgroup, each with the same bits, since each reads it back)
+    qkv_prologue<D, KVT, G>(a, hu, part == nparts - 1, s_q, tid, ctx_raw);
   } else {
     load_q(a.q + head0 * D, D);
   }
@@ -590,6 +620,7 @@ __global__ __launch_bounds__(kThreads) void decode_partition_kernel(DecodeArgs a
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   if (tid == 0) {
+    const int unit = (SHARES ? blockIdx.y * pairs : 0) + pair;
     const unsigned arrived =
         __hip_atomic_fetch_add(&a.counters[unit], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
     s_last = arrived == static_cast<unsigned>(nparts);
@@ -597,7 +628,7 @@ __global__ __launch_bounds__(kThreads) void decode_partition_kernel(DecodeArgs a
   }
   __syncthreads();
   if (!s_last) return;
-  merge_unit<D, G, true>(a, head0, nparts, s_w, s_inv);
+  merge_unit<D, G, true>(a, head0, group, nparts, s_w, s_inv);
 }
 
 // The separate merge launch (used where the partition kernel does not merge): one workgroup
@@ -608,14 +639,12 @@ __global__ __launch_bounds__(kThreads) void decode_merge_kernel(DecodeArgs a) {
   constexpr int kPartTokens = kWaves * WT;
   __shared__ float s_w[MAXG][kMaxParts];
   __shared__ float s_inv[MAXG];
-  const int pair = blockIdx.x;
-  const int seq = pair / a.hkv;
-  const int kvh = pair % a.hkv;
-  const int ctx = min(a.context_lens[seq], a.parts_per_seq * kPartTokens);  // clamped as in the partitions
+  const HeadUnit u = head_unit<true>(a, blockIdx.x);
+  if (u.heads <= 0) return;
+  const int ctx = min(a.context_lens[u.seq], a.parts_per_seq * kPartTokens);  // clamped as in the partitions
   const int nparts = (ctx + kPartTokens - 1) / kPartTokens;
   if (nparts <= 1) return;
-  const size_t head0 = (size_t)seq * a.hq + (size_t)kvh * a.group;
-  merge_unit<D, MAXG, false>(a, head0, nparts, s_w, s_inv);
+  merge_unit<D, MAXG, false>(a, u.head0, u.heads, nparts, s_w, s_inv);
 }
 
 // One workgroup per token: copies the token's [Hkv, D] K and V rows into their pool slot.
@@ -775,17 +804,24 @@ int32_t zero_async(fi_context* ctx, void* p, size_t bytes) {
 }
 
 template <int D, typename KVT, int G>
-int32_t launch_decode_group(fi_context* ctx, const DecodeArgs& args, unsigned grid, int wt) {
-  if (wt == FI_DECODE_WIDE_WAVE_TOKENS) {
-    hipLaunchKernelGGL((decode_partition_kernel<D, KVT, G, FI_DECODE_WIDE_WAVE_TOKENS>), dim3(grid), dim3(kThreads), 0,
-                       ctx->stream, args);
-  } else {
-    hipLaunchKernelGGL((decode_partition_kernel<D, KVT, G, FI_DECODE_NARROW_WAVE_TOKENS>), dim3(grid), dim3(kThreads),
-                       0, ctx->stream, args);
-  }
+int32_t launch_decode_group(fi_context* ctx, const DecodeArgs& args, dim3 grid, int wt) {
+  auto launch = [&](auto wave_tokens) {
+    constexpr int WT = decltype(wave_tokens)::value;
+    if constexpr (G < 8) {  // a share holds at most half of 8 heads
+      if (grid.y > 1) {
+        hipLaunchKernelGGL((decode_partition_kernel<D, KVT, G, WT, true>), grid, dim3(kThreads), 0, ctx->stream, args);
+        return;
+      }
+    }
+    hipLaunchKernelGGL((decode_partition_kernel<D, KVT, G, WT, false>), grid, dim3(kThreads), 0, ctx->stream, args);
+  };
+  if (wt == FI_DECODE_WIDE_WAVE_TOKENS)
+    launch(std::integral_constant<int, FI_DECODE_WIDE_WAVE_TOKENS>{});
+  else
+    launch(std::integral_constant<int, FI_DECODE_NARROW_WAVE_TOKENS>{});
   FI_CHECK_LAUNCH("decode_partition_kernel");
   if (args.parts_per_seq > 1 && args.counters == nullptr) {
-    const dim3 grid2(static_cast<unsigned>(args.num_seqs) * args.hkv);
+    const dim3 grid2(static_cast<unsigned>(args.num_seqs) * args.hkv, grid.y);
     if (wt == FI_DECODE_WIDE_WAVE_TOKENS) {
       hipLaunchKernelGGL((decode_merge_kernel<D, G, FI_DECODE_WIDE_WAVE_TOKENS>), grid2, dim3(kThreads), 0, ctx->stream,
                          args);
@@ -799,16 +835,18 @@ int32_t launch_decode_group(fi_context* ctx, const DecodeArgs& args, unsigned gr
 }
 
 template <int D, typename KVT>
-int32_t launch_decode(fi_context* ctx, const DecodeArgs& args, unsigned grid, int wt) {
-  if (args.group <= 1) return launch_decode_group<D, KVT, 1>(ctx, args, grid, wt);
-  if (args.group <= 2) return launch_decode_group<D, KVT, 2>(ctx, args, grid, wt);
-  if (args.group <= 4) return launch_decode_group<D, KVT, 4>(ctx, args, grid, wt);
-  if (args.group <= 8) return launch_decode_group<D, KVT, 8>(ctx, args, grid, wt);
+int32_t launch_decode(fi_context* ctx, const DecodeArgs& args, dim3 grid, int wt) {
+  if (args.group <= 8) {
+    if (args.heads_per <= 1) return launch_decode_group<D, KVT, 1>(ctx, args, grid, wt);
+    if (args.heads_per <= 2) return launch_decode_group<D, KVT, 2>(ctx, args, grid, wt);
+    if (args.heads_per <= 4) return launch_decode_group<D, KVT, 4>(ctx, args, grid, wt);
+    return launch_decode_group<D, KVT, 8>(ctx, args, grid, wt);
+  }
   return fi::set_error(FI_ERR_UNSUPPORTED, "decode attention supports at most 8 query heads per KV head");
 }
 
 template <int D>
-int32_t launch_decode_dtype(fi_context* ctx, int32_t dtype, const DecodeArgs& args, unsigned grid, int wt) {
+int32_t launch_decode_dtype(fi_context* ctx, int32_t dtype, const DecodeArgs& args, dim3 grid, int wt) {
   if (dtype == FI_DTYPE_F32) return launch_decode<D, float>(ctx, args, grid, wt);
   return launch_decode<D, uint16_t>(ctx, args, grid, wt);
 }
@@ -971,6 +1009,21 @@ int32_t fi_kv_gather(fi_context* ctx, const void* d_k_cache, const void* d_v_cac
 
 namespace {
 
+// Workgroups that share a (sequence, kv head, partition), each over some of the group's heads.  A
+// launch of few workgroups is bound by one workgroup's serial chain, most of it arithmetic in
+// proportion to its heads, so it is cut by heads while the chip has room: each share reads the
+// same K/V (through one L2, see head_unit) and computes its heads exactly as the whole group's
+// workgroup would, so outputs do not depend on the cut.  In two while that leaves two workgroups
+// per CU, in four while it leaves one (us, 1 / 2 / 4 shares):
+//   7 heads, D 64, f32: 1 sequence of 700 tokens 12.9 / 9.6 / 8.3, 16 of 64-200 9.4 / 7.2 / 6.0,
+//     32 of 64-1000 (256 workgroups) 14.4 / 12.1 / 17.0;
+//   4 heads, D 128, f32: 8 of 200-400 (64 workgroups) 14.3 / 11.4 / 10.1, 16 (128) 14.7 / 11.8 / 13.2;
+//   4 heads, D 128, bf16: 1 of 1000 16.4 / 12.7 / 10.7, 8 of 200-2000 (256) 16.9 / 15.2.
+int head_split(int64_t whole, int group, int64_t cus) {
+  if (group >= 4 && 4 * whole <= cus) return 4;
+  return group >= 2 && 2 * whole <= 2 * cus ? 2 : 1;
+}
+
 // Shared by both decode entry points: validation, launch shape and launches.  With
 // `noalloc` the partials go to the library's fixed scratch array instead of the context
 // workspace (nothing is allocated).
@@ -1082,15 +1135,18 @@ int32_t decode_paged(fi_context* ctx, const float* d_q, const void* d_k_cache, c
       FI_TRY(fi::decode_scratch(ctx, num_seqs, num_q_heads, parts, head_dim, &args.part_acc, &args.part_ml));
     }
   }
-  const unsigned grid = static_cast<unsigned>(num_seqs) * num_kv_heads * parts;
+  const int64_t cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
+  const int64_t whole = static_cast<int64_t>(num_seqs) * num_kv_heads * parts;  // workgroups with whole groups
+  const int shares = head_split(whole, args.group, cus);
+  args.heads_per = (args.group + shares - 1) / shares;
+  const dim3 grid(static_cast<unsigned>(whole), static_cast<unsigned>(shares));
   // Small launches (at most six workgroups a CU, e.g. a decode tick of a small model) merge
   // in the last-arriving partition workgroup: the separate merge launch's fixed cost is a large
   // share there (C4 tick at batch 64: 2.375 against 2.403-2.410 ms).  Large launches keep the
   // separate merge, where the merging workgroups' tail costs more than the launch (C2, 2048
   // workgroups: 113.2 against 111.4 us).
-  const int64_t cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
   if (parts > 1 && !noalloc && ctx->d_merge_counters != nullptr &&
-      static_cast<int64_t>(num_seqs) * num_kv_heads <= FI_MERGE_COUNTERS && static_cast<int64_t>(grid) <= 6 * cus)
+      static_cast<int64_t>(num_seqs) * num_kv_heads * shares <= FI_MERGE_COUNTERS && whole <= 6 * cus)
     args.counters = ctx->d_merge_counters;
   switch (head_dim) {
     case 32:

@@ -475,3 +475,54 @@ def test_decode_fused_qkv_matches_consumer_then_decode(gpu_ctx, kv_dtype, case):
         assert torch.equal(q2, q1)
     else:
         assert torch.isnan(q2).all()  # the fused kernel leaves q_out unwritten
+
+
+@pytest.mark.parametrize("kv_dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("hq,hkv,d", [(7, 1, 64), (14, 2, 64), (5, 1, 32), (8, 2, 32), (6, 2, 128), (32, 8, 128),
+                                      (2, 1, 64), (8, 8, 64)])
+def test_decode_head_shares_do_not_change_outputs(gpu_ctx, kv_dtype, hq, hkv, d):
+    """A launch of few workgroups cuts each query-head group into two or four shares (uneven ones,
+    and an empty one, among these groups); a large launch does not.  A sequence's output is the
+    same bits in all of them, plain and fused with the q|k|v consumer, as are the pools."""
+    import torch
+
+    from ferrisinfer_amd import DTYPE_BF16, DTYPE_F32
+
+    print(f"head shares {hq}/{hkv} d={d} {kv_dtype}", flush=True)
+    bs, dt = 16, DTYPE_F32 if kv_dtype == "f32" else DTYPE_BF16
+    lens = np.array([700, 33, 1, 16, 513, 256, 257, 300] + [40] * (max(8, 600 // hkv) - 8), np.int32)
+    n, width, splits = len(lens), (hq + 2 * hkv) * d, 2
+    nblk = (lens + bs - 1) // bs
+    tables = np.zeros((n, int(nblk.max())), np.int32)
+    order, at = np.random.default_rng(hq + d).permutation(int(nblk.sum())).astype(np.int32), 0
+    for i, k in enumerate(nblk):
+        tables[i, :k] = order[at:at + k]
+        at += k
+    g = torch.Generator(device="cuda").manual_seed(hq * d)
+    normal = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    pools = [normal(at, hkv, bs, d).to(torch.float32 if kv_dtype == "f32" else torch.bfloat16) for _ in range(2)]
+    q, parts = normal(n, hq, d), normal(splits, n, width)
+    cos_t, sin_t = normal(700, d // 2), normal(700, d // 2)
+    pos = lens - 1
+    slots = np.array([int(tables[i, p // bs]) * bs + p % bs for i, p in enumerate(pos)], np.int64)
+
+    def run(rows):
+        k, v = pools[0].clone(), pools[1].clone()
+        m = len(rows)
+        bt, cl = _dev(np.ascontiguousarray(tables[rows]), torch), _dev(np.ascontiguousarray(lens[rows]), torch)
+        plain, fused = (torch.full((m, hq, d), float("nan"), device="cuda") for _ in range(2))
+        top = int(lens[rows].max())
+        gpu_ctx.attn_decode_paged(q[rows].contiguous(), k, v, dt, bt, cl, top, hkv, bs, at, d ** -0.5, plain)
+        gpu_ctx.attn_decode_paged_qkv(parts[:, rows].contiguous(), splits, None, _dev(pos[rows].astype(np.int32), torch),
+                                      cos_t, sin_t, d, 700, _dev(slots[rows], torch), k, v, dt, bt, cl, top, hq, hkv,
+                                      d, bs, at, d ** -0.5, fused, q_out=torch.empty(m, hq, d, device="cuda"))
+        return plain, fused, k, v
+
+    whole = run(np.arange(n))
+    for few in (1, 8, min(n, max(8, 128 // (hkv * 3))), min(n, max(8, 256 // (hkv * 3)))):
+        got = run(np.arange(few))
+        assert torch.equal(got[0], whole[0][:few]) and torch.equal(got[1], whole[1][:few]), few
+        used = torch.from_numpy(slots[:few]).cuda()
+        for a, b in zip(got[2:], whole[2:]):
+            assert torch.equal(a[used // bs, :, used % bs], b[used // bs, :, used % bs])
+    gpu_ctx.check_faults()

@@ -423,18 +423,17 @@ __device__ __forceinline__ void split3(const f32x8& x, bf16x8& hi, bf16x8& mid, 
   lo = __builtin_bit_cast(bf16x8, l);
 }
 
-__device__ __forceinline__ v4f mfma_s3(const bf16x8& ah, const bf16x8& am, const bf16x8& al, const bf16x8& bh,
-                                       const bf16x8& bm, const bf16x8& bl, v4f acc) {
-  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh, acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl, acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am, bm, acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am, bh, acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bm, acc, 0, 0, 0);
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh, acc, 0, 0, 0);
-}
+// The six cross products above 2^-24 relative, smallest first: piece indices (a, b) into
+// (hi, mid, lo).
+constexpr int kTermA[6] = {2, 0, 1, 1, 0, 0};
+constexpr int kTermB[6] = {0, 2, 1, 0, 1, 0};
 
+// Three workgroups a CU (168 registers, 48 KiB of LDS each): counters of two showed the MFMAs busy
+// 34 % of the time, the split's VALU work 29 % and the waves waiting for the rest, so a third wave
+// a SIMD fills in (w1|w3 at 914 rows 134 -> 122 us, the 64-row greedy head 170 -> 156 us,
+// 200 rows 583 -> 538 us).  The K-tail form would spill there and keeps two.
 template <int MT, int PW, int EPI, bool KTAIL>
-__global__ __launch_bounds__(kThreads, 2) void gemm_s3_kernel(PGemmArgs g) {
+__global__ __launch_bounds__(kThreads, KTAIL ? 2 : 3) void gemm_s3_kernel(PGemmArgs g) {
   using BV = typename PVec<PW>::T;
   constexpr int KC = 2;                 // 32-k steps per staged A chunk
   constexpr int R = 2 * KC;             // B ring slots span two chunks: slot of step j of chunk c = (c % 2) KC + j
@@ -443,7 +442,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_s3_kernel(PGemmArgs g) {
   constexpr int F_PER_T = (FRAGS + kThreads - 1) / kThreads;
   __shared__ bf16x8 s_a[2][3][FRAGS];
 
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: the slab's address needs no VGPRs
   const int slab_id = blockIdx.x * kWaves + w;
   const int slab = min(slab_id, g.slabs - 1);  // a short last group still loads valid data
   const int m0 = blockIdx.y * 16 * MT, z = blockIdx.z;
@@ -517,6 +517,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_s3_kernel(PGemmArgs g) {
       issue_b(s + DEPTH, (cs * KC + j + DEPTH) % R);
       sched_fence();
       if (s < nsteps) {
+        bf16x8 b[PW][3];
 #pragma unroll
         for (int p = 0; p < PW; ++p) {
           const int slot = cs * KC + j;
@@ -524,14 +525,22 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_s3_kernel(PGemmArgs g) {
                            PVec<PW>::get(rb[slot][0][2], p), PVec<PW>::get(rb[slot][0][3], p),
                            PVec<PW>::get(rb[slot][1][0], p), PVec<PW>::get(rb[slot][1][1], p),
                            PVec<PW>::get(rb[slot][1][2], p), PVec<PW>::get(rb[slot][1][3], p)};
-          bf16x8 bh, bm, bl;
-          split3(x, bh, bm, bl);
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt) {
-            const int f = (j * MT + mt) * 64 + lane;
-            acc[mt][p] = mfma_s3(sa[f], sa[FRAGS + f], sa[2 * FRAGS + f], bh, bm, bl, acc[mt][p]);
-          }
+          split3(x, b[p][0], b[p][1], b[p][2]);
         }
+        bf16x8 a[MT][3];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int t = 0; t < 3; ++t) a[mt][t] = sa[t * FRAGS + (j * MT + mt) * 64 + lane];
+        // term by term over the tiles: a tile's six products depend on each other, so each waits
+        // behind the other tiles' instead of its own predecessor
+#pragma unroll
+        for (int t = 0; t < 6; ++t)
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int p = 0; p < PW; ++p)
+              acc[mt][p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt][kTermA[t]], b[p][kTermB[t]], acc[mt][p], 0, 0, 0);
       }
       sched_fence();
     }
@@ -565,15 +574,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_s3_kernel(PGemmArgs g) {
 // no barrier in the loop; the quarters are summed through LDS in wave order, and workgroups
 // along z split K further (partials [splits, M, N], summed by the consumers in split order).
 typedef float v16f __attribute__((ext_vector_type(16)));
-
-__device__ __forceinline__ void mfma_x32(v16f& acc, const bf16x8 (&a)[3], const bf16x8 (&b)[3]) {
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], b[0], acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[2], acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[1], acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[0], acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[1], acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], acc, 0, 0, 0);
-}
 
 __device__ __forceinline__ void split3_pair(const float4& x0, const float4& x1, bf16x8 (&p)[3]) {
   const f32x8 x = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
@@ -636,9 +636,13 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_w32_kernel(PGemmArgs g) {
 #pragma unroll
           for (int s = 0; s < SL; ++s) split3_pair(rw[d][s][0], rw[d][s][1], pw[s]);
 #pragma unroll
-          for (int t = 0; t < MT; ++t)
+          for (int x = 0; x < 6; ++x)  // term by term over the tiles, as in gemm_s3_kernel
 #pragma unroll
-            for (int s = 0; s < SL; ++s) mfma_x32(acc[t][s], pa[t], pw[s]);
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+              for (int s = 0; s < SL; ++s)
+                acc[t][s] =
+                    __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[t][kTermA[x]], pw[s][kTermB[x]], acc[t][s], 0, 0, 0);
         }
         sched_fence();
       }

@@ -52,7 +52,8 @@ struct PrefillArgs {
   float scale;
   int num_seqs;
   int max_query_len;
-  const int* order;          // (sequence, query tile) pairs, largest first
+  const int* order;          // (sequence, query tile) pairs, largest first; null: tile_of's own order
+  int fold;                  // that order pairs long and short tiles (see prefill_plan_kernel)
   // prefill_x3_kernel with key splits: each (tile, kv head) runs as kv_splits workgroups over
   // consecutive ranges of its key chunks, writing partials (unnormalised O, reference point and
   // row sum per row) that prefill_split_merge_kernel combines in split order
@@ -110,6 +111,27 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(const int* __restric
   }
 }
 
+// The tile (seq * ntiles + query tile) of a rank.  Without a planned order: one sequence's tiles
+// from its last to its first, which is largest first, folded as the plan folds them; several
+// sequences' last tiles, then the ones before, and so on (launches of at most one workgroup a CU).
+__device__ __forceinline__ int tile_of(const PrefillArgs& a, int rank, int ntiles, int qt_tokens) {
+  if (a.order) return a.order[rank];
+  if (a.num_seqs > 1) {
+    const int t = rank / a.num_seqs;
+    return (rank - t * a.num_seqs) * ntiles + ntiles - 1 - t;
+  }
+  const int n = min(ntiles, (a.cu_seqlens[1] - a.cu_seqlens[0] + qt_tokens - 1) / qt_tokens);
+  if (rank >= n) return rank;  // past the sequence's end
+  const int half = (n + 1) / 2;
+  return a.fold && rank >= half ? rank - half : n - 1 - rank;
+}
+
+// What the plan reports, where there is none: a query length beyond the tiles that max_query_len
+// sized (its tail rows get no workgroup).
+__device__ __forceinline__ void check_query_length(const PrefillArgs& a, int qt, int qlen, int rows) {
+  if (!a.order && qt == 0 && qlen > rows && threadIdx.x == 0) atomicOr(a.faults, FI_FAULT_QUERY_RANGE);
+}
+
 // Four consecutive K/V elements of one row as raw registers, widened when staged.
 template <typename KVT>
 struct Quad;
@@ -155,10 +177,11 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_kernel(PrefillArgs a) {
   // keeps to one kv head's K/V (Hkv = 8) or a fixed subset of heads.
   const int ntiles = (a.max_query_len + QT - 1) / QT;
   const int rank = blockIdx.x / a.hkv, kvh = blockIdx.x % a.hkv;
-  const int tile = a.order[rank];
+  const int tile = tile_of(a, rank, ntiles, QT);
   const int qt = tile % ntiles, seq = tile / ntiles;
   const int qs = a.cu_seqlens[seq];
   const int qlen = a.cu_seqlens[seq + 1] - qs;
+  check_query_length(a, qt, qlen, ntiles * QT);
   const int q0 = qt * QT;
   if (q0 >= qlen) return;
   const int ctx = a.context_lens[seq];
@@ -370,8 +393,13 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_kernel(PrefillArgs a) {
   }
 }
 
-// Sorts the tiles largest first into the context workspace (one small launch before the
-// attention kernel) and sizes the grid: one workgroup per (tile, kv head).
+// Sizes the grid (one workgroup per tile and kv head, and split) and sorts the tiles largest first
+// into the context workspace, one small launch before the attention kernel (4.7 us).  No plan
+// where the kernels know as good an order: a single sequence, and several whose workgroups
+// have a CU each (13 prompts of 20-70 tokens, 14/2 heads: 12.1 -> 8.2 us; a 2048-token chunk
+// after 2048, bf16: 130.6 -> 126.5 us; 700 tokens after 300, f32 pool: 71.5 -> 67.5 us).  At two to
+// four a CU the unplanned order cost more than the launch (3 sequences of 20-150 tokens after up
+// to 2000, 32/8 heads, f32 pool: 104 planned, 118 us without).
 #ifndef FI_PREFILL_FOLD
 #define FI_PREFILL_FOLD 1
 #endif
@@ -380,22 +408,27 @@ int32_t plan_tiles(fi_context* ctx, PrefillArgs& args, int qt, int kb, const cha
                    size_t part_floats = 0) {
   const int ntiles = (args.max_query_len + qt - 1) / qt;
   const long pairs = (long)ntiles * args.num_seqs;
-  FI_REQUIRE(pairs * args.hkv * splits <= 0x7fffffffL, FI_ERR_INVALID_SHAPE, std::string(name) + ": grid too large");
+  const long wgs = pairs * args.hkv * splits;
+  FI_REQUIRE(wgs <= 0x7fffffffL, FI_ERR_INVALID_SHAPE, std::string(name) + ": grid too large");
+  const long cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
+  const bool plan = args.num_seqs > 1 && wgs > cus;
   // the tile order, then (split launches) each workgroup's partials
-  const size_t order_bytes = ((size_t)pairs * sizeof(int) + 255) & ~static_cast<size_t>(255);
-  const size_t part_bytes = splits > 1 ? (size_t)pairs * args.hkv * splits * part_floats * sizeof(float) : 0;
-  FI_TRY(fi::ensure_workspace(ctx, order_bytes + part_bytes));
-  int* order = static_cast<int*>(ctx->workspace);
+  const size_t order_bytes = plan ? ((size_t)pairs * sizeof(int) + 255) & ~static_cast<size_t>(255) : 0;
+  const size_t part_bytes = splits > 1 ? (size_t)wgs * part_floats * sizeof(float) : 0;
+  if (order_bytes + part_bytes > 0) FI_TRY(fi::ensure_workspace(ctx, order_bytes + part_bytes));
   args.kv_splits = splits;
   args.part = splits > 1 ? reinterpret_cast<float*>(static_cast<char*>(ctx->workspace) + order_bytes) : nullptr;
   // one round of workgroups (two per CU): pair long and short tiles on each CU
-  const long cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
-  const int fold = FI_PREFILL_FOLD && splits == 1 && pairs * args.hkv <= 2 * cus;
-  hipLaunchKernelGGL(prefill_plan_kernel, dim3(1), dim3(1024), 0, ctx->stream, args.cu_seqlens, args.context_lens,
-                     args.num_seqs, ntiles, qt, kb, fold, order, ctx->d_faults);
-  FI_CHECK_LAUNCH("prefill_plan_kernel");
-  args.order = order;
-  *grid = dim3(static_cast<unsigned>(pairs * args.hkv * splits));
+  args.fold = FI_PREFILL_FOLD && splits == 1 && wgs <= 2 * cus;
+  args.order = nullptr;
+  if (plan) {
+    int* order = static_cast<int*>(ctx->workspace);
+    hipLaunchKernelGGL(prefill_plan_kernel, dim3(1), dim3(1024), 0, ctx->stream, args.cu_seqlens, args.context_lens,
+                       args.num_seqs, ntiles, qt, kb, args.fold, order, ctx->d_faults);
+    FI_CHECK_LAUNCH("prefill_plan_kernel");
+    args.order = order;
+  }
+  *grid = dim3(static_cast<unsigned>(wgs));
   return FI_OK;
 }
 
@@ -483,10 +516,11 @@ __global__ __launch_bounds__(kThreads, FI_PREFILL_BF16_WAVES) void prefill_bf16_
   const uint16_t* __restrict__ v_cache = static_cast<const uint16_t*>(a.v_cache);
   const int ntiles = (a.max_query_len + QT - 1) / QT;
   const int rank = blockIdx.x / a.hkv, kvh = blockIdx.x % a.hkv;
-  const int tile = a.order[rank];
+  const int tile = tile_of(a, rank, ntiles, QT);
   const int qt = tile % ntiles, seq = tile / ntiles;
   const int qs = a.cu_seqlens[seq];
   const int qlen = a.cu_seqlens[seq + 1] - qs;
+  check_query_length(a, qt, qlen, ntiles * QT);
   const int q0 = qt * QT;
   if (q0 >= qlen) return;
   const int ctx = a.context_lens[seq];
@@ -810,10 +844,11 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_x3_kernel(PrefillArgs a) 
   const int wg = blockIdx.x / a.hkv, kvh = blockIdx.x % a.hkv;
   const int rank = SPLIT ? wg / a.kv_splits : wg;
   const int split = SPLIT ? wg - rank * a.kv_splits : 0;
-  const int tile = a.order[rank];
+  const int tile = tile_of(a, rank, ntiles, QT);
   const int qt = tile % ntiles, seq = tile / ntiles;
   const int qs = a.cu_seqlens[seq];
   const int qlen = a.cu_seqlens[seq + 1] - qs;
+  check_query_length(a, qt, qlen, ntiles * QT);
   const int q0 = qt * QT;
   if (q0 >= qlen) return;
   const int ctx = a.context_lens[seq];

@@ -438,3 +438,51 @@ def test_prefill_query_beyond_max_query_len_reported(gpu_ctx):
     torch.cuda.synchronize()
     gpu_ctx.check_faults()
     assert torch.equal(out[:20], solo)
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(14, 2, 64), (32, 8, 128), (8, 2, 32)])
+@pytest.mark.parametrize("kv", ["f32", "bf16", "bf16-mfma"])
+def test_prefill_order_without_plan(gpu_ctx, hq, hkv, d, kv):
+    """Launches with and without the planning launch: one sequence (folded and unfolded order, a
+    max_query_len well past its length), sequences that together leave a CU per workgroup and ones
+    that do not.  Every row against f64 (1e-5 normwise over an f32-math path, whose error is a few
+    f32 roundings; 1e-2 where queries and probabilities are rounded to bf16); a sequence alone
+    gives what it gives beside others within the same bounds."""
+    import torch
+
+    from ferrisinfer_amd import DTYPE_BF16, DTYPE_F32
+
+    print(f"prefill order {hq}/{hkv} d={d} {kv}", flush=True)
+    bs, g = 16, torch.Generator(device="cuda").manual_seed(d + hq)
+    dt = torch.float32 if kv == "f32" else torch.bfloat16
+    for seqs, slack in (([(37, 200)], 0), ([(37, 200)], 300), ([(0, 1)], 0), ([(64, 1500)], 0),
+                        ([(5, 9), (0, 17), (33, 30)], 4), ([(100, 90), (0, 160), (7, 200), (0, 33)], 0)):
+        lens = [p + n for p, n in seqs]
+        nblk = [-(-x // bs) for x in lens]
+        tables = torch.zeros(len(seqs), max(nblk), dtype=torch.int32, device="cuda")
+        order, at = torch.randperm(sum(nblk), generator=g, device="cuda").int(), 0
+        for i, k in enumerate(nblk):
+            tables[i, :k] = order[at:at + k]
+            at += k
+        k, v = (torch.randn(at, hkv, bs, d, generator=g, device="cuda").to(dt) for _ in range(2))
+        cu = np.concatenate([[0], np.cumsum([n for _, n in seqs])]).astype(np.int32)
+        q = torch.randn(int(cu[-1]), hq, d, generator=g, device="cuda")
+        out = torch.full_like(q, float("nan"))
+        args = (tables, torch.from_numpy(cu).cuda(), torch.tensor(lens, dtype=torch.int32, device="cuda"),
+                max(n for _, n in seqs) + slack, hkv, bs, at, d ** -0.5, out)
+        if kv == "bf16-mfma":
+            gpu_ctx.attn_prefill_paged_bf16(q, k, v, *args)
+        else:
+            gpu_ctx.attn_prefill_paged(q, k, v, DTYPE_F32 if kv == "f32" else DTYPE_BF16, *args)
+        want = torch.empty_like(q, dtype=torch.float64)
+        for i, (p, n) in enumerate(seqs):
+            ids = tables[i, :nblk[i]].long()
+            keys, vals = (x[ids].transpose(1, 2).reshape(-1, hkv, d)[:p + n].double() for x in (k, v))
+            mask = torch.arange(p + n, device="cuda")[None] > p + torch.arange(n, device="cuda")[:, None]
+            for h in range(hq):
+                j = h // (hq // hkv)
+                s = (q[cu[i]:cu[i + 1], h].double() @ keys[:, j].t()) * d ** -0.5
+                want[cu[i]:cu[i + 1], h] = torch.softmax(s.masked_fill(mask, float("-inf")), dim=1) @ vals[:, j]
+        err = ((out.double() - want).norm() / want.norm()).item()
+        assert err <= (1e-2 if kv == "bf16-mfma" else 1e-5), (seqs, err)
+    gpu_ctx.check_faults()

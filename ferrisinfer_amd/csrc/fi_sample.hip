@@ -8,8 +8,9 @@
 // keeps the list's values equal to the k largest values of the prefix scanned so far, so:
 //   * fast path, one pass: a logit below the k+1-th largest value of some part of the row
 //     cannot be among the k + 1 largest.  Each wave buffers in LDS only the logits at or above
-//     its running bound (the k+1-th largest of what it has buffered, raised to the other
-//     waves' bounds) and compacts the buffer by radix selection when it fills.  When the k+1
+//     its running bound (seeded from the maxima of the workgroup's threads over its first
+//     steps, then the k+1-th largest of what it has buffered, raised to the other waves'
+//     bounds) and compacts the buffer by radix selection when it fills.  When the k+1
 //     largest values of the row are strictly decreasing and the row holds no NaN, the final
 //     list is exactly the k largest logits, in value order.  With equal values among them the
 //     list still holds the same values in the same sorted order (equal values, equal weights),
@@ -26,7 +27,7 @@
 // reserves (fi_sample_reserve): a radix sort of the row's candidates and sequential walks over
 // the sorted weights, with the same replay, over a tree of list minima, for a shared drawn
 // value.
-// Weights exp(l / T - l0 / T) are computed in parallel; one lane then forms the total, the
+// Weights exp(l / T - l0 / T) are computed in parallel; one wave then forms the total, the
 // top-p prefix, the retained total, the xorshift64* draw and the threshold walk, sequentially
 // in f32 in list order.  The exponential is the device expf; the reference's is the host
 // libm's, so a weight may differ in its last bit.
@@ -45,6 +46,7 @@ constexpr int kStep = 64 * kPerLane;  // logits per wave step
 constexpr int kGroup = 256;           // logits per wave appended between buffer checks
 constexpr int kRegion = 1536;         // buffered candidates per wave: k + 1 (at most 1025), equal ones, one group
 constexpr int kSortMax = 2048;        // fast-path candidates sorted at the end
+constexpr int kSelectHeld = 2048;     // a selection over at most this many holds them in registers
 constexpr int kRankSortMax = 256;     // at most this many: rank counting, else a bitonic sort
 constexpr int kIntMin = static_cast<int>(0x80000000u);
 
@@ -97,45 +99,38 @@ __device__ __forceinline__ void load_step(const float* row, int vocab, int s, in
   }
 }
 
-// Runs f(logits, s) over wave steps first, first + stride, ... with a ring of four step
-// buffers (the first three primed by prime_steps with the same range): three steps of loads
-// are in flight while one is processed.  Every call is made
-// unconditionally (steps at or past nsteps hold no real logit; f masks them by index) so that
-// no load is sunk into a branch next to its use.  Those steps load step nsteps - 1 again, which
-// the range has just read, instead of the logits past the range (another segment's, which
-// would be read from memory twice).
-// The ring's first three steps, loaded by prime_steps before the row's configuration is read
-// (the loads do not depend on it), so the configuration's round trip overlaps them.
+// Wave steps first, first + stride, ... go through a ring of kRing step buffers.  prime_steps
+// fills it before the row's configuration is read (the loads do not depend on it, so the
+// configuration's round trip overlaps them); stream_steps runs f(logits, s) over the same range,
+// reloading each buffer as f leaves it.  Every call is made unconditionally (steps at or past
+// nsteps hold no real logit; f masks them by index) so that no load is sunk into a branch next
+// to its use.  Those steps load step nsteps - 1 again, which the range has just read, instead
+// of the logits past the range (another segment's, which would be read from memory twice).
+// Four buffers: three primed ones leave the bound below a quarter fewer logits, five spill
+// (64 rows of 151936, top-k 20: 21.2 us with four, 21.9 with five).
+constexpr int kRing = 4;
 struct StepRing {
-  float b0[kPerLane], b1[kPerLane], b2[kPerLane];
+  float b[kRing][kPerLane];
 };
 
 template <int VEC>
 __device__ __forceinline__ void prime_steps(const float* row, int vocab, int first, int stride, int nsteps, int lane,
                                             StepRing& ring) {
   const int last = max(nsteps - 1, 0);
-  load_step<VEC>(row, vocab, min(first, last), lane, ring.b0);
-  load_step<VEC>(row, vocab, min(first + stride, last), lane, ring.b1);
-  load_step<VEC>(row, vocab, min(first + 2 * stride, last), lane, ring.b2);
+#pragma unroll
+  for (int j = 0; j < kRing; ++j) load_step<VEC>(row, vocab, min(first + j * stride, last), lane, ring.b[j]);
 }
 
 template <int VEC, typename F>
 __device__ __forceinline__ void stream_steps(const float* row, int vocab, int first, int stride, int nsteps, int lane,
                                              StepRing& ring, F&& f) {
   const int last = max(nsteps - 1, 0);
-  float(&b0)[kPerLane] = ring.b0;
-  float(&b1)[kPerLane] = ring.b1;
-  float(&b2)[kPerLane] = ring.b2;
-  float b3[kPerLane];
-  for (int s = first; s < nsteps; s += 4 * stride) {
-    load_step<VEC>(row, vocab, min(s + 3 * stride, last), lane, b3);
-    f(b0, s);
-    load_step<VEC>(row, vocab, min(s + 4 * stride, last), lane, b0);
-    f(b1, s + stride);
-    load_step<VEC>(row, vocab, min(s + 5 * stride, last), lane, b1);
-    f(b2, s + 2 * stride);
-    load_step<VEC>(row, vocab, min(s + 6 * stride, last), lane, b2);
-    f(b3, s + 3 * stride);
+  for (int s = first; s < nsteps; s += kRing * stride) {
+#pragma unroll
+    for (int j = 0; j < kRing; ++j) {
+      f(ring.b[j], s + j * stride);
+      load_step<VEC>(row, vocab, min(s + (j + kRing) * stride, last), lane, ring.b[j]);
+    }
   }
 }
 
@@ -310,7 +305,7 @@ struct SampleShared {
   } u;
   float s_val[kMaxTopK + 1];  // the sorted list
   int s_idx[kMaxTopK + 1];
-  alignas(16) float wts[kMaxTopK];  // its weights (zero past k)
+  alignas(16) float wts[kMaxTopK];  // its weights (zero past k, to a multiple of kWalkBlock)
   int bound[kWaves];    // each wave's current lower bound (a total_cmp key)
   int count[kWaves];
   int flags;  // bit 0: NaN seen, bit 1: buffer overflow, bit 2: not strictly decreasing
@@ -583,6 +578,72 @@ __device__ __forceinline__ GreedyPart greedy_pass(const float* row, int vocab, i
   return g;
 }
 
+// The largest t with more than k of the wave's 64 * N keys at or above t, built bit by bit from
+// the top, one ballot a key and bit (0 when no more than k keys are above it).
+template <int N>
+__device__ __forceinline__ uint32_t rank_bound(const uint32_t (&u)[N], int k) {
+  uint32_t t = 0;
+#pragma unroll
+  for (int b = 31; b >= 0; --b) {
+    const uint32_t c = t | (1u << b);
+    int n = 0;
+#pragma unroll
+    for (int q = 0; q < N; ++q) n += __popcll(__ballot(u[q] >= c));
+    t = n > k ? c : t;
+  }
+  return t;
+}
+
+// A lower bound of the segment's k+1-th largest key, from the steps in the ring (whole
+// workgroup): the (k+1)-th largest of its threads' maxima.  k+1 distinct logits lie at or above
+// it, so nothing below it can be among the k+1 largest.  The ring covers up to 32768 logits, so
+// the bound is close to their k+1-th largest: at 64 rows of 151936 a segment buffers about 25
+// logits for k = 20, where a bound from each wave's first step let ~730 through to an exact
+// radix selection (both launches 27.8 -> 21.2 us; 257 rows 85 -> 55 us).  Below k = 64 it is
+// taken from 128 maxima of four threads each (two ballots a bit instead of eight).
+template <int VEC>
+__device__ __forceinline__ int seed_bound(const StepRing& ring, int s0, int s1, int lim, int k, int w, int lane,
+                                          bool whole, SampleShared& sh) {
+  int lmax = kIntMin;
+#pragma unroll
+  for (int j = 0; j < kRing; ++j) {
+    const int s = s0 + w + j * kWaves;
+    const int valid = s < s1 ? lim - s * kStep : 0;
+    if (valid >= kStep) {  // a NaN among them marks the row in the pass, whatever the bound
+      float top = ring.b[j][0];
+#pragma unroll
+      for (int e = 1; e < kPerLane; ++e) top = __builtin_elementwise_maximum(top, ring.b[j][e]);
+      lmax = max(lmax, total_key(top));
+    } else if (valid > 0) {
+#pragma unroll
+      for (int e = 0; e < kPerLane; ++e) {
+        lmax = max(lmax, step_index<VEC>(0, lane, e) < valid ? total_key(ring.b[j][e]) : kIntMin);
+      }
+    }
+  }
+  if (whole && k < kWaves && s1 - s0 <= kWaves) {
+    // a short row and few wanted: a bound per wave from its own step lets no more through than
+    // is ranked at once, and needs no barrier (4096 logits, top-k 2: 8.5 against 9.1 us)
+    const uint32_t own[1] = {static_cast<uint32_t>(lmax) ^ 0x80000000u};
+    return static_cast<int>(rank_bound<1>(own, k) ^ 0x80000000u);
+  }
+  sh.u.fast.key[w * 64 + lane] = lmax;  // unused until the pass is over
+  __syncthreads();
+  uint32_t u[kWaves];
+#pragma unroll
+  for (int q = 0; q < kWaves; ++q) u[q] = static_cast<uint32_t>(sh.u.fast.key[q * 64 + lane]) ^ 0x80000000u;
+  uint32_t t;
+  if (k < 64) {
+    uint32_t h[2] = {u[0], u[1]};
+#pragma unroll
+    for (int q = 2; q < kWaves; ++q) h[q & 1] = max(h[q & 1], u[q]);
+    t = rank_bound<2>(h, k);
+  } else {
+    t = rank_bound<kWaves>(u, k);
+  }
+  return static_cast<int>(t ^ 0x80000000u);
+}
+
 // One pass over wave steps [s0, s1) (logit indices below lim): each wave buffers in its LDS
 // region the logits that can be among the k+1 largest of what the workgroup has seen (whole
 // workgroup).  Leaves sh.count[w] and sets sh.flags bit 0 (NaN) / bit 1 (a region overflowed
@@ -592,33 +653,17 @@ __device__ __forceinline__ void buffer_pass(const float* row, int vocab, int s0,
                             SampleShared& sh, StepRing& ring) {
   int* rkey = sh.key[w];
   int* ridx = sh.idx[w];
-  int bound = kIntMin, cnt = 0;
+  // seeded while k is below half of the threads that hold logits; nearer to all of them the
+  // bound is close to the smallest maximum and filters little
+  int bound = kIntMin;
+  if (k < 32 * min(kWaves, s1 - s0)) {
+    bound = seed_bound<VEC>(ring, s0, s1, lim, k, w, lane, s0 == 0 && lim == vocab, sh);
+  }
+  int cnt = 0;
   uint32_t nan_bits = 0;  // max of |bits|: above 0x7f800000 when a NaN was seen
   stream_steps<VEC>(row, vocab, s0 + w, kWaves, s1, lane, ring, [&](const float (&v)[kPerLane], int s) {
     const int valid = lim - s * kStep;  // logits of this step below lim: step_index offsets < valid
     if (valid <= 0) return;             // a ring slot past the segment (wave-uniform)
-    if (k < 64 && s < s0 + kWaves) {
-      // the wave's first step seeds its bound: the (k+1)-th largest of the 64 lane maxima.
-      // k+1 distinct logits of the step are at or above it, so nothing below it can be among
-      // the k+1 largest (empty lanes hold the minimum key).  It is the largest t with at least
-      // k+1 lane maxima at or above t, built bit by bit from the top over order-preserving
-      // unsigned keys, one ballot a bit.  Later steps raise the bound by compaction.
-      int lmax = kIntMin;
-#pragma unroll
-      for (int e = 0; e < kPerLane; ++e)
-        lmax = max(lmax, step_index<VEC>(0, lane, e) < valid ? total_key(v[e]) : kIntMin);
-      const uint32_t u = static_cast<uint32_t>(lmax) ^ 0x80000000u;
-      uint32_t t = 0;
-#pragma unroll
-      for (int b = 31; b >= 0; --b) {
-        const uint32_t c = t | (1u << b);
-        t = __popcll(__ballot(u >= c)) > k ? c : t;
-      }
-      bound = max(bound, static_cast<int>(t ^ 0x80000000u));
-      // published at once, so the other waves filter their later steps against it too (the
-      // wave buffers the k+1 logits that make it valid in this step)
-      if (lane == 0) atomicMax(&sh.bound[w], bound);
-    }
     int hits = 0;
     if (valid >= kStep) {
       // a whole step: its NaN-propagating maximum (-0 below +0) decides whether any logit
@@ -681,7 +726,7 @@ __device__ __forceinline__ int select_desc(SampleShared& sh, int rank, int tid, 
   // Up to kOwn candidates a thread (flattened over the wave buffers) are read into registers
   // once, so each round's histogram is a few compares and increments instead of a loop whose
   // bounds and keys are LDS reads; larger sets read the buffers every round.
-  constexpr int kOwn = 4;
+  constexpr int kOwn = kSelectHeld / kThreads;
   int cnt[kWaves];
   int total = 0;
 #pragma unroll
@@ -757,12 +802,10 @@ __device__ __forceinline__ bool fast_top_k(SampleShared& sh, int k, int tid, int
     // few candidates (every buffer holds more than k of them together): all of them go to the
     // rank sort, whose order is total, so no selection round is needed
     int base = 0;
-    for (int q = 0; q < kWaves; ++q) {
-      for (int i = tid; i < sh.count[q]; i += kThreads) {
-        sh.u.fast.key[base + i] = sh.key[q][i];
-        sh.u.fast.idx[base + i] = sh.idx[q][i];
-      }
-      base += sh.count[q];
+    for (int q = 0; q < w; ++q) base += sh.count[q];
+    for (int i = lane; i < sh.count[w]; i += 64) {
+      sh.u.fast.key[base + i] = sh.key[w][i];
+      sh.u.fast.idx[base + i] = sh.idx[w][i];
     }
     if (tid == 0) sh.m = total;
   } else {
@@ -784,14 +827,22 @@ __device__ __forceinline__ bool fast_top_k(SampleShared& sh, int k, int tid, int
   if (m > kSortMax) return false;
   // ---- ranks 0..k by (key descending, index ascending) ----
   if (m <= kRankSortMax) {
-    for (int i = tid; i < m; i += kThreads) {
-      const int key = sh.u.fast.key[i], id = sh.u.fast.idx[i];
-      int rank = 0;
-      for (int j = 0; j < m; ++j) rank += before(sh.u.fast.key[j], sh.u.fast.idx[j], key, id);
-      if (rank <= k) {
-        sh.s_val[rank] = key_value(key);
-        sh.s_idx[rank] = id;
+    // 2, 4 or 8 adjacent threads count a candidate's rank, each over its share of the others
+    const int lg = m <= 64 ? 3 : m <= 128 ? 2 : 1;
+    const int i = tid >> lg, share = 1 << lg;
+    const bool in = i < m;
+    const int key = in ? sh.u.fast.key[i] : 0, id = in ? sh.u.fast.idx[i] : 0;
+    int rank = 0;
+    if (in) {
+#pragma unroll 8
+      for (int j = tid & (share - 1); j < m; j += share) {
+        rank += before(sh.u.fast.key[j], sh.u.fast.idx[j], key, id);
       }
+    }
+    for (int off = 1; off < share; off <<= 1) rank += __shfl_xor(rank, off, 64);
+    if (in && (tid & (share - 1)) == 0 && rank <= k) {
+      sh.s_val[rank] = key_value(key);
+      sh.s_idx[rank] = id;
     }
   } else {
     block_bitonic_sort(sh.u.fast.key, sh.u.fast.idx, m, tid);
@@ -802,9 +853,8 @@ __device__ __forceinline__ bool fast_top_k(SampleShared& sh, int k, int tid, int
   }
   __syncthreads();
   for (int i = tid; i < k; i += kThreads) {
-    if (!(sh.s_val[i] > sh.s_val[i + 1])) atomicOr(&sh.flags, 4);
+    if (!(sh.s_val[i] > sh.s_val[i + 1])) atomicOr(&sh.flags, 4);  // read after weights_and_draw's barriers
   }
-  __syncthreads();
   return true;
 }
 
@@ -864,94 +914,110 @@ __device__ __forceinline__ void replay_sorted(const float* row, int vocab, int k
   __syncthreads();
 }
 
-// Weights (parallel), then the total, top-p, draw and threshold walk (one lane, in the
-// reference's sequential f32 order) over the sorted list s_val / s_idx of k candidates.  Leaves
-// the drawn list position in sh.draw and writes the probability, or faults the row (sh.draw
-// -1).  Every thread returns after the closing barrier.
-// SamplerState::next_f32 (sampler.rs:62-75): advances rng[r] and returns the draw.
-__device__ __forceinline__ float next_draw(uint64_t* rng, int r) {
-  const uint64_t x = xorshift_step(rng[r]);
-  rng[r] = x;
+// SamplerState::next_f32 (sampler.rs:62-75): the draw of an advanced state.
+__device__ __forceinline__ float unit_draw(uint64_t x) {
   const uint32_t upper = static_cast<uint32_t>((x * 0x2545F4914F6CDD1DULL) >> 40);
   return static_cast<float>(upper) / 16777216.0f;
 }
 
+constexpr int kWalkBlock = 16;  // weights per block of the walks: at most 64 blocks, one sum a lane
+static_assert(kMaxTopK <= 64 * kWalkBlock && kMaxTopK % kWalkBlock == 0, "one block sum per lane");
+
 // The total, top-p prefix, draw and threshold walk of sampler.rs:190-233 over k weights in
-// list order (one lane; wts 16-byte aligned and zero from k to the next multiple of 8).  The
-// top-p loop's running sum repeats the total's additions in the same order from the same +0,
-// so the retained total, summed again from the start by the reference, is the running sum
-// where that loop stops.  Returns the drawn position and writes the probability, or faults the
-// row and returns -1.
-__device__ __forceinline__ int draw_one(const float* wts, int k, float P, uint64_t* rng, int32_t* token, float* prob,
-                                        uint32_t* faults, int r) {
+// list order (one wave, every lane the same; wts 16-byte aligned and zero from k to the next
+// multiple of kWalkBlock).  The top-p loop's running sum repeats the total's additions in the
+// same order from the same +0, so the retained total, summed again from the start by the
+// reference, is the running sum where that loop stops.  Neither sum ever falls and the
+// threshold never rises, so the walks run a block at a time, its weights loaded together, and
+// only the block where a value crosses is walked again one weight at a time: top-k 255 of 4096
+// logits, one row, 29.6 -> 22.2 us against loads of 4 or 8 weights and a test at each.
+// Returns the drawn position and writes the probability, or faults the row and returns -1.
+__device__ __forceinline__ int draw_one(const float* wts, int k, float P, uint64_t state, uint64_t* rng, int32_t* token,
+                                        float* prob, uint32_t* faults, int r, int lane) {
 #pragma clang fp contract(off)
-  const float4* w4 = reinterpret_cast<const float4*>(wts);  // + 0.0f past k leaves a sum >= +0 unchanged
-  float total = 0.0f;
-  for (int i = 0; i < k; i += 8) {
-    const float4 a = w4[i / 4], b = w4[i / 4 + 1];
-    total = total + a.x;
-    total = total + a.y;
-    total = total + a.z;
-    total = total + a.w;
-    total = total + b.x;
-    total = total + b.y;
-    total = total + b.z;
-    total = total + b.w;
+  const auto load = [&](int at, float(&t)[kWalkBlock]) {
+#pragma unroll
+    for (int q = 0; q < kWalkBlock / 4; ++q) {
+      const float4 a = reinterpret_cast<const float4*>(wts + at)[q];
+      t[4 * q] = a.x;
+      t[4 * q + 1] = a.y;
+      t[4 * q + 2] = a.z;
+      t[4 * q + 3] = a.w;
+    }
+  };
+  const int blocks = (k + kWalkBlock - 1) / kWalkBlock;
+  float t[kWalkBlock];
+  float total = 0.0f, ends = 0.0f;  // lane b: the running sum after block b
+  for (int b = 0; b < blocks; ++b) {
+    load(b * kWalkBlock, t);
+#pragma unroll
+    for (int j = 0; j < kWalkBlock; ++j) total = total + t[j];  // + 0.0f past k leaves a sum >= +0 unchanged
+    ends = lane == b ? total : ends;
   }
   if (!(total <= 3.402823466e+38f) || total <= 0.0f) {  // not finite, or no mass
-    sampling_fault(faults, FI_FAULT_SAMPLE_NONFINITE, token, prob, r);
+    if (lane == 0) sampling_fault(faults, FI_FAULT_SAMPLE_NONFINITE, token, prob, r);
     return -1;
   }
   float p = P;  // f32::clamp(0, 1): a NaN stays NaN
   if (p < 0.0f) p = 0.0f;
   if (p > 1.0f) p = 1.0f;
   const float cutoff = p >= 1.0f ? total : total * p;
-  float kept = 0.0f;
-  int retained = 0;
-  for (int i = 0; i < k; i += 4) {
-    const float4 a = w4[i / 4];
-    const float t[4] = {a.x, a.y, a.z, a.w};
-    bool reached = false;
+  float kept = total;
+  int retained = k;
+  const uint64_t crossed = __ballot(lane < blocks && ends >= cutoff);
+  if (crossed != 0) {  // always, but for a NaN cutoff
+    const int b = __builtin_ctzll(crossed);
+    kept = b > 0 ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ends), b - 1)) : 0.0f;
+    load(b * kWalkBlock, t);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (!reached && i + j < k) {
-        kept = kept + t[j];
-        ++retained;
-        reached = kept >= cutoff;
+    for (int j = 0; j < kWalkBlock; ++j) {
+      kept = kept + t[j];
+      if (kept >= cutoff) {  // reached within k: the sums past it repeat the last
+        retained = b * kWalkBlock + j + 1;
+        break;
       }
     }
-    if (reached) break;
   }
-  const float retained_total = kept;  // retained >= 1: the loop adds at least one weight
-  float threshold = next_draw(rng, r) * retained_total;
+  const uint64_t x = xorshift_step(state);
+  if (lane == 0) rng[r] = x;
+  float threshold = unit_draw(x) * kept;
   int sel = 0;
-  for (int i = 0; i < retained; i += 4) {
-    const float4 a = w4[i / 4];
-    const float t[4] = {a.x, a.y, a.z, a.w};
-    bool hit = false;
+  for (int at = 0; at < retained; at += kWalkBlock) {
+    load(at, t);
+    float end = threshold;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (!hit && i + j < retained) {
+    for (int j = 0; j < kWalkBlock; ++j) end = end - t[j];
+    if (end <= 0.0f) {
+#pragma unroll
+      for (int j = 0; j < kWalkBlock; ++j) {
         threshold = threshold - t[j];
         if (threshold <= 0.0f) {
-          sel = i + j;
-          hit = true;
+          if (at + j < retained) sel = at + j;
+          break;
         }
       }
+      break;
     }
-    if (hit) break;
+    threshold = end;
   }
-  prob[r] = wts[sel] / retained_total;
+  if (lane == 0) prob[r] = wts[sel] / kept;
   return sel;
 }
 
-__device__ __forceinline__ void weights_and_draw(SampleShared& sh, int k, float T, float P, uint64_t* rng,
-                                                 int32_t* token, float* prob, uint32_t* faults, int r, int tid) {
+// Weights (parallel), then the total, top-p, draw and threshold walk (one wave, in the
+// reference's sequential f32 order) over the sorted list s_val / s_idx of k candidates.  Leaves
+// the drawn list position in sh.draw and writes the probability, or faults the row (sh.draw
+// -1).  Every thread returns after the closing barrier.
+__device__ __forceinline__ void weights_and_draw(SampleShared& sh, int k, float T, float P, uint64_t state,
+                                                 uint64_t* rng, int32_t* token, float* prob, uint32_t* faults, int r, int tid) {
   const float temp = fmaxf(T, 1.1920929e-7f);  // max(f32::EPSILON); a NaN temperature gives EPSILON
   const float scaled_max = sh.s_val[0] / temp;
-  for (int i = tid; i < kMaxTopK; i += kThreads) sh.wts[i] = i < k ? weight_exp((sh.s_val[i] / temp) - scaled_max) : 0.0f;
+  for (int i = tid; i < (k + kWalkBlock - 1) / kWalkBlock * kWalkBlock; i += kThreads) sh.wts[i] = i < k ? weight_exp((sh.s_val[i] / temp) - scaled_max) : 0.0f;
   __syncthreads();
-  if (tid == 0) sh.draw = draw_one(sh.wts, k, P, rng, token, prob, faults, r);
+  if (tid < 64) {
+    const int sel = draw_one(sh.wts, k, P, state, rng, token, prob, faults, r, tid);
+    if (tid == 0) sh.draw = sel;
+  }
   __syncthreads();
 }
 
@@ -1010,8 +1076,24 @@ __global__ __launch_bounds__(kThreads) void sample_scan_kernel(const float* __re
   int* okey = cand_key + ((size_t)r * segs + seg) * kRegion;
   int* oidx = cand_idx + ((size_t)r * segs + seg) * kRegion;
   if (sh.flags == 0) {
-    // the segment's k+1-th largest (every buffered logit when the segment holds at most k+1)
-    const int kth = total > k + 1 ? select_desc(sh, k, tid, w, lane) : kIntMin;
+    // All of them, with no selection here, where they are few enough that the finish ranks every
+    // segment's directly, or where it has a selection to do in any case (the k + 1 of every
+    // segment reach its limit) and holds that many in registers.
+    const int direct = (k + 1) * segs >= kRankSortMax ? kSelectHeld / segs : kRankSortMax / segs;
+    if (total <= max(k + 1, direct)) {
+      int base = 0;
+      for (int q = 0; q < w; ++q) base += sh.count[q];
+      for (int i = lane; i < sh.count[w]; i += 64) {
+        okey[base + i] = sh.key[w][i];
+        oidx[base + i] = sh.idx[w][i];
+      }
+      if (tid == 0) {
+        out->count = total;
+        out->flags = 0;
+      }
+      return;
+    }
+    const int kth = select_desc(sh, k, tid, w, lane);  // the segment's k+1-th largest
     for (int q = 0; q < kWaves; ++q) {
       for (int i = tid; i < sh.count[q]; i += kThreads) {
         if (sh.key[q][i] >= kth) {
@@ -1048,6 +1130,7 @@ __global__ __launch_bounds__(kThreads) void sample_finish_kernel(
   const float T = temperature[r];
   const int K = top_k[r];
   const float P = top_p[r];
+  const uint64_t state = rng[r];  // read here, not in a round trip of its own at the draw
   const ScanMeta* rm = meta + (size_t)r * segs;
 
   if (greedy_row(T, K, P)) {
@@ -1109,9 +1192,21 @@ __global__ __launch_bounds__(kThreads) void sample_finish_kernel(
         sh.key[w][lane] = key0;
         sh.idx[w][lane] = idx0;
       }
-      for (int i = lane + 64; i < c; i += 64) {
-        sh.key[w][i] = ck[i];
-        sh.idx[w][i] = ci[i];
+      for (int base = 64; base < c; base += 256) {  // four loads of each at once (clamped, stored below c)
+        int bk[4], bi[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          bk[j] = ck[min(base + 64 * j + lane, c - 1)];
+          bi[j] = ci[min(base + 64 * j + lane, c - 1)];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int i = base + 64 * j + lane;
+          if (i < c) {
+            sh.key[w][i] = bk[j];
+            sh.idx[w][i] = bi[j];
+          }
+        }
       }
     }
     if (lane == 0) sh.count[w] = c;
@@ -1120,7 +1215,7 @@ __global__ __launch_bounds__(kThreads) void sample_finish_kernel(
   }
 
   if (!sorted) replay_sorted<VEC>(row, vocab, k, tid, w, lane, sh);
-  weights_and_draw(sh, k, T, P, rng, token, prob, faults, r, tid);
+  weights_and_draw(sh, k, T, P, state, rng, token, prob, faults, r, tid);
   write_token<VEC>(sh, row, vocab, k, sorted, token, r, tid, w, lane);
 }
 
@@ -1143,6 +1238,7 @@ __global__ __launch_bounds__(kThreads) void sample_row_kernel(const float* __res
   const float T = temperature[r];
   const int K = top_k[r];
   const float P = top_p[r];
+  const uint64_t state = rng[r];
   const int nsteps = (vocab + kStep - 1) / kStep;
   StepRing ring;
   prime_steps<VEC>(row, vocab, w, kWaves, nsteps, lane, ring);
@@ -1171,7 +1267,7 @@ __global__ __launch_bounds__(kThreads) void sample_row_kernel(const float* __res
     if (sh.flags == 0) sorted = fast_top_k(sh, k, tid, w, lane);
   }
   if (!sorted) replay_sorted<VEC>(row, vocab, k, tid, w, lane, sh);
-  weights_and_draw(sh, k, T, P, rng, token, prob, faults, r, tid);
+  weights_and_draw(sh, k, T, P, state, rng, token, prob, faults, r, tid);
   write_token<VEC>(sh, row, vocab, k, sorted, token, r, tid, w, lane);
 }
 
@@ -1715,7 +1811,8 @@ __global__ __launch_bounds__(kThreads) void sample_large_kernel(const float* __r
     });
   }
   if (tid == 0) {
-    sh.thr = next_draw(rng, r) * sh.rtotal;
+    rng[r] = xorshift_step(rng[r]);
+    sh.thr = unit_draw(rng[r]) * sh.rtotal;
     sh.sel = 0;
     sh.wsel = wt.of(wt.value(0));
   }

@@ -153,6 +153,31 @@ def test_sample_tokens_plateau_at_the_boundary(orc, gpu_ctx, plateau):
         states = new_states
 
 
+@pytest.mark.parametrize("vocab,pad,copies", [(1023, 0, 1), (2048, 0, 1), (4096, 0, 1), (8193, 0, 12), (9216, 0, 12),
+                                              (33000, 0, 1), (70001, 2, 1)])
+def test_sample_tokens_seeded_bound(orc, gpu_ctx, vocab, pad, copies):
+    """The scan's bound comes from its threads' maxima: top-k on both sides of each of its forms
+    (a wave's own, 128 maxima, 512, none), rows of one to eight segments, and rows whose largest
+    logits all lie with a few threads (every 64th float4 or scalar), ascend or descend."""
+    print(f"sample seeded bound vocab={vocab}", flush=True)
+    rng = np.random.default_rng(vocab)
+    configs = [(0.8, k, p) for k in (2, 7, 8, 31, 32, 63, 64, 127, 128, 255, 256) for p in (0.95,)] * copies
+    states = [orc.sampler_state_new(300 + i) for i in range(len(configs))]
+    lanes = np.arange(vocab) // (4 if vocab % 4 == 0 and pad == 0 else 1) % 64
+    for layout in ("random", "one lane", "ascending", "descending"):
+        logits = (rng.standard_normal((len(configs), vocab)) * 2.0).astype(np.float32)
+        if layout == "one lane":
+            logits[:, lanes == 5] += np.float32(12.0)
+        elif layout != "random":
+            logits = np.sort(logits, axis=1)
+            if layout == "descending":
+                logits = np.ascontiguousarray(logits[:, ::-1])
+        tok, prob, new_states = run_device(gpu_ctx, padded_logits(logits, pad), configs, states)
+        gpu_ctx.check_faults()
+        check_rows(orc, logits, configs, states, tok, prob, new_states, layout)
+        states = new_states
+
+
 def test_sample_tokens_c5_head_shape(orc, gpu_ctx):
     """257 rows x 128256 (the Llama-3-8B head's batch in the C5 step) under chat_default and
     greedy rows."""

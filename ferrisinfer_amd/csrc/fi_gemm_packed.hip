@@ -861,14 +861,21 @@ using fi::sum_splits;
 constexpr int kRowThreads = 256;  // of the row-wise consumers
 // THREADS is kRowThreads, or kWideRowThreads where the rows are wide and no more than one a CU: a
 // thread then holds one float4 of a 4096-wide row instead of four, a quarter of the dependent
-// split-load rounds (16 rows x 4096: 18.8 us with 32 splits before, 6.0 us with 7).
+// split-load rounds (7 splits: 256 rows x 4096 9.9 -> 7.7 us, 16 x 8192 10.2 -> 7.3, 64 x 16384
+// 27.8 -> 14.4; 257 rows x 4096 take 10.2 us).  The sum of squares is taken by the first kRowThreads
+// threads over the same quads in the same order in both, from LDS in the wide form, so a row's
+// bits do not depend on how many rows the call has.  Widths that are no multiple of four, or past
+// what the wide form holds in registers, stay narrow.
 constexpr int kWideRowThreads = 1024;
+constexpr int kRowQuads = 8;  // float4 a thread keeps between the two passes
 template <int THREADS, bool OUT16>
 __global__ __launch_bounds__(THREADS) void splitk_residual_rms_norm_kernel(
     const float* __restrict__ parts, int splits, const float* __restrict__ bias, const float* __restrict__ residual,
     float* __restrict__ sum_out, const float* __restrict__ weight, void* __restrict__ out_v, int rows, int hidden,
     float eps) {
-  __shared__ float s_red[THREADS / 64];
+  constexpr bool WIDE = THREADS > kRowThreads;  // held rows only
+  __shared__ float s_red[kRowThreads / 64];
+  __shared__ float4 s_x[WIDE ? THREADS : 1];
   const int row = blockIdx.x;
   const size_t plane = (size_t)rows * hidden;
   const size_t base = (size_t)row * hidden;
@@ -876,20 +883,24 @@ __global__ __launch_bounds__(THREADS) void splitk_residual_rms_norm_kernel(
   const bool vec = (hidden & 3) == 0;
   // rows up to kRowQuads float4 per thread keep their sums in registers for the second pass
   // (no re-read of sum_out); wider rows loop and re-read
-  constexpr int kRowQuads = 8;
   const int h4 = hidden / 4;
-  const bool held = vec && h4 <= kRowQuads * THREADS;
+  const bool held = WIDE || (vec && h4 <= kRowQuads * THREADS);
   float4 xs[kRowQuads];
   float4 ws[kRowQuads];  // held rows: the norm weights, loaded with the partials (one memory round trip)
+  // fused by name: left to the compiler, which of the first two squares is rounded by itself can
+  // differ between the two forms
+  auto square_quad = [&](const float4& x) {
+    ss = fmaf(x.x, x.x, ss);
+    ss = fmaf(x.y, x.y, ss);
+    ss = fmaf(x.z, x.z, ss);
+    ss = fmaf(x.w, x.w, ss);
+  };
   auto sum_quad = [&](int c) {
     float4 x = sum_splits(reinterpret_cast<const float4*>(parts + base) + c, plane / 4, splits);
     if (bias) x = add(x, reinterpret_cast<const float4*>(bias)[c]);
     x = add(x, reinterpret_cast<const float4*>(residual + base)[c]);
     reinterpret_cast<float4*>(sum_out + base)[c] = x;
-    ss += x.x * x.x;
-    ss += x.y * x.y;
-    ss += x.z * x.z;
-    ss += x.w * x.w;
+    if constexpr (!WIDE) square_quad(x);
     return x;
   };
   if (held) {
@@ -903,6 +914,20 @@ __global__ __launch_bounds__(THREADS) void splitk_residual_rms_norm_kernel(
       const int c = threadIdx.x + i * THREADS;
       if (c < h4) xs[i] = sum_quad(c);
     }
+    if constexpr (WIDE) {
+#pragma unroll
+      for (int i = 0; i < kRowQuads; ++i) {
+        if (i * THREADS >= h4) break;  // uniform
+        if (i > 0) __syncthreads();
+        s_x[threadIdx.x] = xs[i];
+        __syncthreads();
+        if (threadIdx.x < kRowThreads) {
+#pragma unroll
+          for (int j = 0; j < THREADS; j += kRowThreads)
+            if (i * THREADS + j + static_cast<int>(threadIdx.x) < h4) square_quad(s_x[j + threadIdx.x]);
+        }
+      }
+    }
   } else if (vec) {
     for (int c = threadIdx.x; c < h4; c += THREADS) (void)sum_quad(c);
   } else {
@@ -915,11 +940,11 @@ __global__ __launch_bounds__(THREADS) void splitk_residual_rms_norm_kernel(
     }
   }
   ss = fi::wave_sum(ss);
-  if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = ss;
+  if ((threadIdx.x & 63) == 0 && threadIdx.x < kRowThreads) s_red[threadIdx.x >> 6] = ss;
   __syncthreads();
   float total = 0.0f;
 #pragma unroll
-  for (int i = 0; i < THREADS / 64; ++i) total += s_red[i];
+  for (int i = 0; i < kRowThreads / 64; ++i) total += s_red[i];
   const float inv = 1.0f / sqrtf(total / static_cast<float>(hidden) + eps);
   // OUT16: the normalised row is stored as bf16 bits, each value rounded to nearest even
   float* out = static_cast<float*>(out_v);
@@ -958,7 +983,8 @@ template <bool OUT16>
 void launch_row_norm(fi_context* ctx, const float* parts, int splits, const float* bias, const float* residual,
                      float* sum, const float* weight, void* out, int rows, int hidden, float eps) {
   const int cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
-  if (hidden >= 2048 && rows <= cus)
+  const bool held = hidden % 4 == 0 && hidden / 4 <= kRowQuads * kWideRowThreads;
+  if (hidden >= 2048 && rows <= cus && held)
     hipLaunchKernelGGL((splitk_residual_rms_norm_kernel<kWideRowThreads, OUT16>), dim3(rows), dim3(kWideRowThreads),
                        0, ctx->stream, parts, splits, bias, residual, sum, weight, out, rows, hidden, eps);
   else

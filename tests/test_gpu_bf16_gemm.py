@@ -367,3 +367,30 @@ def test_residual_norm_wide_rows(gpu_ctx, rows):
         normed = want / (want.square().mean(dim=1, keepdim=True) + 1e-6).sqrt() * w.double()
         for got, exact in ((total, want), (out, normed)):
             assert ((got.double() - exact).norm() / exact.norm()).item() <= 1e-6
+
+
+@pytest.mark.parametrize("hidden", [2048, 4096, 4100, 4101, 8192, 12292, 32768, 32772])
+def test_residual_norm_row_bits_do_not_depend_on_row_count(gpu_ctx, hidden):
+    """Calls of up to one row a CU take wide workgroups, larger ones narrow workgroups: a row of
+    the same partials has the same bits in both, f32 and bf16, with and without a bias."""
+    import torch
+
+    print(f"residual norm row bits hidden={hidden}", flush=True)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    g = torch.Generator(device="cuda").manual_seed(hidden)
+    normal = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    n = cus + 1
+    parts, res, w, bias = normal(2, n, hidden), normal(n, hidden), normal(hidden), normal(hidden)
+
+    def run(rows, dtype, b):
+        total, out = torch.empty(rows, hidden, device="cuda"), torch.empty(rows, hidden, device="cuda", dtype=dtype)
+        gpu_ctx.splitk_residual_rms_norm(parts[:, :rows].contiguous(), 2, b, res[:rows].contiguous(), total, w, out,
+                                         1e-6)
+        return total, out
+
+    for dtype in (torch.float32, torch.bfloat16):
+        for b in (None, bias):
+            whole = run(n, dtype, b)
+            for rows in (1, 33, cus):
+                for few, many in zip(run(rows, dtype, b), whole):
+                    assert torch.equal(few, many[:rows]), (dtype, rows)

@@ -178,6 +178,26 @@ def test_sample_tokens_seeded_bound(orc, gpu_ctx, vocab, pad, copies):
         states = new_states
 
 
+@pytest.mark.parametrize("vocab", [61, 255, 1000, 1024, 1025, 1500, 2047])
+def test_sample_tokens_few_steps(orc, gpu_ctx, vocab):
+    """Rows of one and two wave steps: top-k on both sides of each choice of bound (a wave's own, the
+    workgroup's, none), with the largest logits spread out, with one lane, and repeated."""
+    print(f"sample few steps vocab={vocab}", flush=True)
+    rng = np.random.default_rng(vocab)
+    configs = [(0.8, k, 0.95) for k in (2, 7, 8, 15, 16, 31, 32, 48, 59, 60)]
+    states = [orc.sampler_state_new(700 + i) for i in range(len(configs))]
+    for layout in ("random", "one lane", "equal"):
+        logits = (rng.standard_normal((len(configs), vocab)) * 2.0).astype(np.float32)
+        if layout == "one lane":
+            logits[:, np.arange(vocab) // 4 % 64 == 5] += np.float32(12.0)
+        elif layout == "equal":
+            logits = np.round(logits)
+        tok, prob, new_states = run_device(gpu_ctx, padded_logits(logits, 0), configs, states)
+        gpu_ctx.check_faults()
+        check_rows(orc, logits, configs, states, tok, prob, new_states, layout)
+        states = new_states
+
+
 def test_sample_tokens_c5_head_shape(orc, gpu_ctx):
     """257 rows x 128256 (the Llama-3-8B head's batch in the C5 step) under chat_default and
     greedy rows."""

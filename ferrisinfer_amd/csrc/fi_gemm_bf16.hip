@@ -496,6 +496,8 @@ __global__ __launch_bounds__(64 * SW * KW, 2) void gemm_bf16_rows_kernel(BGemmAr
 
 int32_t q_steps(int32_t k) { return (k + kStepK - 1) / kStepK; }
 
+int num_cus(fi_context* ctx) { return ctx->compute_units > 0 ? ctx->compute_units : 256; }
+
 constexpr int kNt = 4;  // slabs per wave: a workgroup covers 256 columns
 
 constexpr int kRowsMax = 64;   // gemm_bf16_rows_kernel up to this many rows
@@ -523,10 +525,11 @@ int rows_slabs(int slabs) { return slabs >= 256 ? 8 : 4; }
 template <int MT, int EPI, bool A16>
 void launch_rows_mt(fi_context* ctx, const BGemmArgs& g) {
   if constexpr (EPI == kEpiSwiglu) {
-    // one launch without partials; a workgroup takes eight slabs where that still gives 128 of
-    // them (1792 slabs: 42.5 us against 54 us with four slabs and K in four parts), else four
-    // (608 slabs, 64 rows: 9.2 us against 13.2 us with eight)
-    if (g.slabs >= 1024)
+    // one launch without partials; a workgroup takes eight slabs where four would be more than a
+    // workgroup per CU (1056 slabs, K 2048, 64 rows: 23.6 us against 31.0 us with four slabs and K
+    // in four parts), else four (1024 slabs: 18.7 us against 23.1 us with eight; 608, K 896: 9.4
+    // against 12.6)
+    if (g.slabs > 4 * num_cus(ctx))
       launch_rows_as<MT, 2, 4, 2, EPI, A16>(ctx, g);
     else
       launch_rows_as<MT, 2, 2, 4, EPI, A16>(ctx, g);
@@ -555,7 +558,7 @@ int32_t launch_rows(fi_context* ctx, const BGemmArgs& g, bool a16) {
 // measured no better (16 rows, K 14336, 256 slabs: 23.2 against 22.1 us) and their consumer reads
 // twice the partials.
 int rows_splits(fi_context* ctx, int q, int slabs) {
-  const int cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
+  const int cus = num_cus(ctx);
   const int groups = (slabs + rows_slabs(slabs) - 1) / rows_slabs(slabs);
   const int unit = kRowsStage * kRowsParts;
   const int stages = (q + unit - 1) / unit;
@@ -565,6 +568,25 @@ int rows_splits(fi_context* ctx, int q, int slabs) {
   const int s = (q + per - 1) / per;
   const int even = (q + s - 1) / s;
   return (q + even - 1) / even;  // every split non-empty
+}
+
+// Whether SwiGLU of m rows takes gemm_bf16_rows_kernel.  It does not split K over workgroups, so a
+// workgroup's chain of K steps (longer the more rows it stages, f32 rows above all) has to be short,
+// or the slabs enough to fill the chip; the tile kernel splits K.  us, this kernel / tiles with
+// their split sum, f32 rows:
+//   chain at most 2048: 64 rows, K 256, 32 slabs 6.5 / 10.3; 16, K 2048, 64 slabs 8.8 / 9.0;
+//   up to four slabs a CU: 64 rows, K 4096, 512 slabs 41.0 / 27.5, 768 42.7 / 41.9, 896 43.8 /
+//     45.6; 16, K 8192, 128 slabs 33.7 / 15.2, 640 0.88 of tiles; 32, K 2048, 256 slabs 13.4 /
+//     11.1, 640 0.90 of tiles; 64, K 14336, 32 slabs 119 / 16.7;
+//   more: 64 rows, K 5120, 1728 slabs 65.5 / 78.7; 32, K 8192, 1056 slabs 63.4 / 63.0; 64, K 8192,
+//     1056 slabs 92.2 / 82.7, 2752 205 / 179.
+// bf16 rows gain on both sides of the last line (64, K 8192, 1056 slabs 66.8 / 79.1), but the
+// choice is the same for both, so that they give the same bits.
+bool rows_swiglu(fi_context* ctx, int m, int q, int slabs) {
+  if (m > kRowsMax) return false;
+  const int64_t cus = num_cus(ctx), chain = static_cast<int64_t>(q) * (m + 16);
+  if (chain <= 2048) return true;
+  return slabs > 4 * cus ? chain <= 14336 : slabs >= 2 * cus + chain / 40;
 }
 
 #ifndef FI_BGEMM_FORCE_MT
@@ -601,8 +623,7 @@ int mt_for(fi_context* ctx, int m, int slabs) {
 // row-tile K steps, ceil(tiles s / CUs) MT Q / s, at ~67 ns each (16 x 256 x 32 products at the
 // kernel's ~40 % of the bf16 peak per CU), plus each extra partial written and read back at
 // ~6 TB/s (wo at M 2304: 2 splits, 100 -> 83 us with the consumer 23 -> 31 us).
-int split_count(fi_context* ctx, int m, int k, int slabs) {
-  if (m <= kRowsMax) return rows_splits(ctx, q_steps(k), slabs);
+int tile_splits(fi_context* ctx, int m, int k, int slabs) {
   const int mt = mt_for(ctx, m, slabs);
   const int mblocks = (m + 16 * mt - 1) / (16 * mt);
   const int groups = (slabs + kWaves * kNt - 1) / (kWaves * kNt);
@@ -653,21 +674,14 @@ void launch_mt(fi_context* ctx, const BGemmArgs& g, bool a16) {
     launch_mt<MT, EPI, false>(ctx, g);
 }
 
+// The tile kernel.  The greedy head's single K range and its per-tile states suit it at every row
+// count (5 rows x 128256 columns: 182 us against 202 us).
 template <int EPI>
-int32_t launch_bgemm(fi_context* ctx, BGemmArgs g, int splits, bool a16) {
-  // the head's single K range and its per-tile states suit the kernel above at every row count
-  // (5 rows x 128256 columns: 182 us against 202 us)
-  if constexpr (EPI == kEpiPartial || EPI == kEpiSwiglu) {
-    if (g.m <= kRowsMax) {
-      g.splits = splits;
-      return launch_rows<EPI>(ctx, g, a16);
-    }
-  }
+int32_t launch_tiles(fi_context* ctx, BGemmArgs g, bool a16) {
   const int mt = mt_for(ctx, g.m, g.slabs);
   g.mblocks = (g.m + 16 * mt - 1) / (16 * mt);
   g.groups = (g.slabs + kWaves * kNt - 1) / (kWaves * kNt);
-  g.splits = splits;
-  g.total = g.groups * g.mblocks * splits;
+  g.total = g.groups * g.mblocks * g.splits;
   switch (mt) {
     case 8:
       launch_mt<8, EPI>(ctx, g, a16);
@@ -678,13 +692,11 @@ int32_t launch_bgemm(fi_context* ctx, BGemmArgs g, int splits, bool a16) {
     case 4:
       launch_mt<4, EPI>(ctx, g, a16);
       break;
-    default:  // 64 rows or fewer: only the greedy head comes here
-      if constexpr (EPI == kEpiArgmax) {
-        if (mt == 2)
-          launch_mt<2, EPI>(ctx, g, a16);
-        else
-          launch_mt<1, EPI>(ctx, g, a16);
-      }
+    case 2:
+      launch_mt<2, EPI>(ctx, g, a16);
+      break;
+    default:
+      launch_mt<1, EPI>(ctx, g, a16);
       break;
   }
   FI_CHECK_LAUNCH("gemm_bf16_kernel");
@@ -839,7 +851,8 @@ int32_t fi_gemm_bf16_splits(fi_context* ctx, int32_t m, int32_t k, int32_t n, in
   FI_TRY(fi::enter(ctx));
   FI_REQUIRE(m >= 0 && k > 0 && n > 0, FI_ERR_INVALID_SHAPE, "fi_gemm_bf16_splits: bad shape");
   FI_REQUIRE(splits != nullptr, FI_ERR_INVALID_CONFIG, "fi_gemm_bf16_splits: null output");
-  *splits = split_count(ctx, m, k, data_slabs(n, false));
+  const int slabs = data_slabs(n, false);
+  *splits = m <= kRowsMax ? rows_splits(ctx, q_steps(k), slabs) : tile_splits(ctx, m, k, slabs);
   return FI_OK;
 }
 
@@ -863,7 +876,9 @@ int32_t fi_gemm_bf16(fi_context* ctx, const void* d_a, int32_t a_dtype, int32_t 
   const int used = (g.q_total + g.q_per_split - 1) / g.q_per_split;
   FI_REQUIRE(used == splits, FI_ERR_INVALID_CONFIG,
              "fi_gemm_bf16: splits must divide the K steps into non-empty ranges (use fi_gemm_bf16_splits)");
-  return launch_bgemm<kEpiPartial>(ctx, g, splits, a_dtype == FI_DTYPE_BF16);
+  g.splits = splits;
+  const bool a16 = a_dtype == FI_DTYPE_BF16;
+  return m <= kRowsMax ? launch_rows<kEpiPartial>(ctx, g, a16) : launch_tiles<kEpiPartial>(ctx, g, a16);
 }
 
 int32_t fi_gemm_bf16_swiglu(fi_context* ctx, const void* d_a, int32_t a_dtype, int32_t lda, const uint16_t* d_bp_pair,
@@ -886,19 +901,20 @@ int32_t fi_gemm_bf16_swiglu(fi_context* ctx, const void* d_a, int32_t a_dtype, i
   g.lda = lda;
   g.q_total = q_steps(k);
   g.slabs = data_slabs(n, true);
-  const int splits = m <= kRowsMax ? 1 : split_count(ctx, m, k, g.slabs);
-  if (splits == 1) {  // the epilogue applies SwiGLU directly
+  const bool rows = rows_swiglu(ctx, m, g.q_total, g.slabs);
+  g.splits = rows ? 1 : tile_splits(ctx, m, k, g.slabs);
+  if (g.splits == 1) {  // the epilogue applies SwiGLU directly
     g.out = static_cast<float*>(d_out);
     g.out_bf16 = out_dtype == FI_DTYPE_BF16;
     g.q_per_split = g.q_total;
-    return launch_bgemm<kEpiSwiglu>(ctx, g, 1, a16);
+    return rows ? launch_rows<kEpiSwiglu>(ctx, g, a16) : launch_tiles<kEpiSwiglu>(ctx, g, a16);
   }
   // (up, gate) partial pairs per split, then the split sum + SwiGLU
-  FI_TRY(fi::ensure_workspace(ctx, (size_t)splits * m * 2 * n * sizeof(float)));
+  FI_TRY(fi::ensure_workspace(ctx, (size_t)g.splits * m * 2 * n * sizeof(float)));
   g.out = static_cast<float*>(ctx->workspace);
-  g.q_per_split = (g.q_total + splits - 1) / splits;
-  FI_TRY(launch_bgemm<kEpiPairPartial>(ctx, g, splits, a16));
-  return fi::splitk_swiglu(ctx, g.out, splits, d_bias_up, d_bias_gate, m, n, d_out, out_dtype == FI_DTYPE_BF16);
+  g.q_per_split = (g.q_total + g.splits - 1) / g.splits;
+  FI_TRY(launch_tiles<kEpiPairPartial>(ctx, g, a16));
+  return fi::splitk_swiglu(ctx, g.out, g.splits, d_bias_up, d_bias_gate, m, n, d_out, out_dtype == FI_DTYPE_BF16);
 }
 
 int32_t fi_lm_head_argmax_bf16(fi_context* ctx, const void* d_hidden, int32_t a_dtype, int32_t lda,
@@ -920,7 +936,8 @@ int32_t fi_lm_head_argmax_bf16(fi_context* ctx, const void* d_hidden, int32_t a_
   g.tiles = (g.slabs + kNt - 1) / kNt;
   FI_TRY(fi::ensure_workspace(ctx, (size_t)m * g.tiles * 3 * sizeof(float)));
   g.out = static_cast<float*>(ctx->workspace);
-  FI_TRY(launch_bgemm<kEpiArgmax>(ctx, g, 1, a_dtype == FI_DTYPE_BF16));
+  g.splits = 1;
+  FI_TRY(launch_tiles<kEpiArgmax>(ctx, g, a_dtype == FI_DTYPE_BF16));
   return fi::argmax_merge(ctx, g.out, g.tiles, m, d_token, d_prob);
 }
 

@@ -394,3 +394,39 @@ def test_residual_norm_row_bits_do_not_depend_on_row_count(gpu_ctx, hidden):
             for rows in (1, 33, cus):
                 for few, many in zip(run(rows, dtype, b), whole):
                     assert torch.equal(few, many[:rows]), (dtype, rows)
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (1, 4096, 256), (16, 2050, 1024), (48, 1024, 256),     # few slabs behind a long K: split
+    (64, 1024, 4592), (64, 1024, 4608), (33, 4101, 4800),  # both sides of the slabs that fill the chip
+    (16, 64, 8192), (17, 520, 8208),                       # both sides of four slabs a CU
+    (64, 5728, 8208), (64, 5760, 8208)])                   # more slabs, both sides of the longest chain
+def test_bf16_swiglu_few_rows_route(gpu_ctx, m, k, n):
+    """SwiGLU of up to 64 rows on both sides of each choice (one launch over all of K, of four or
+    eight slabs a workgroup, or row tiles with K split): against f64 on the same bf16 operands,
+    whose products are exact in f32, so only the f32 sums differ (1e-5 normwise); f32 and bf16 rows
+    agree bit for bit; with biases, and into bf16, which is the f32 result rounded to nearest even."""
+    import torch
+
+    print(f"bf16 swiglu route m={m} k={k} n={n}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m + k + n)
+    normal = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    a16 = torch.full((m, (k + 7) // 8 * 8), float("nan"), device="cuda", dtype=torch.bfloat16)
+    a16[:, :k] = normal(m, k)
+    w1, w3 = (normal(k, n) * 0.02).bfloat16(), (normal(k, n) * 0.02).bfloat16()
+    bias = normal(2, n) * 0.1
+    pair = gpu_ctx.weight_pack_bf16_pair(w1, w3, k, n)
+    x = a16[:, :k].double()
+    up, gate = x @ w1.double(), x @ w3.double()
+    for b in ((None, None), (bias[0], bias[1])):
+        outs = []
+        for a in (a16, a16.float()):
+            outs.append(torch.full((m, n), float("nan"), device="cuda"))
+            gpu_ctx.gemm_bf16_swiglu(a[:, :k], pair, k, n, outs[-1], *b)
+        assert torch.equal(outs[0], outs[1])
+        want = up * torch.nn.functional.silu(gate) if b[0] is None else \
+            (up + bias[0].double()) * torch.nn.functional.silu(gate + bias[1].double())
+        assert ((outs[0].double() - want).norm() / want.norm()).item() <= 1e-5
+        narrow = torch.empty(m, n, device="cuda", dtype=torch.bfloat16)
+        gpu_ctx.gemm_bf16_swiglu(a16[:, :k], pair, k, n, narrow, *b)
+        assert torch.equal(narrow, outs[0].bfloat16())

@@ -589,6 +589,22 @@ bool rows_swiglu(fi_context* ctx, int m, int q, int slabs) {
   return slabs > 4 * cus ? chain <= 14336 : slabs >= 2 * cus + chain / 40;
 }
 
+// Whether a product of m rows into partials or logits takes gemm_bf16_rows_kernel.  Past half a
+// 256-column group a CU the tile kernel fills the chip without splits and reads the rows once per
+// 256 columns instead of 128; above a group a CU and for few short rows the deeper weight ring
+// still wins.  us, this kernel / tiles, one split:
+//   32000 columns (125 groups), K 4096, f32 rows: 1 row 45.0 / 75.4, 64 rows 62.7 / 86.1;
+//   40000, K 4096: 64 f32 rows 108 / 88.8, 16 f32 67.5 / 78.1, 16 bf16 65.4 / 61.8; 48000, 16 bf16
+//     77.2 / 66.4 (the choice is the same for both, so that they give the same bits);
+//   151936, K 896, f32 rows: 1 row 47.3 / 50.8, 16 53.2 / 52.9, 33 66.0 / 59.0, 64 80.2 / 68.3;
+//   128256, f32 rows: K 1536, 16 rows 72.6 / 72.7; K 2048, 32 rows 102.5 / 97.0; K 4096, 1 row
+//     185.6 / 171.8.
+bool rows_product(fi_context* ctx, int m, int k, int slabs) {
+  if (m > kRowsMax) return false;
+  const int cus = num_cus(ctx), groups = (slabs + kGroupSlabs - 1) / kGroupSlabs;
+  return 2 * groups <= cus || (groups > cus && m <= 16 && k < 2048);
+}
+
 #ifndef FI_BGEMM_FORCE_MT
 #define FI_BGEMM_FORCE_MT 0  // a fixed row tile count above 64 rows (0: chosen per shape)
 #endif
@@ -878,7 +894,8 @@ int32_t fi_gemm_bf16(fi_context* ctx, const void* d_a, int32_t a_dtype, int32_t 
              "fi_gemm_bf16: splits must divide the K steps into non-empty ranges (use fi_gemm_bf16_splits)");
   g.splits = splits;
   const bool a16 = a_dtype == FI_DTYPE_BF16;
-  return m <= kRowsMax ? launch_rows<kEpiPartial>(ctx, g, a16) : launch_tiles<kEpiPartial>(ctx, g, a16);
+  return rows_product(ctx, m, k, g.slabs) ? launch_rows<kEpiPartial>(ctx, g, a16)
+                                          : launch_tiles<kEpiPartial>(ctx, g, a16);
 }
 
 int32_t fi_gemm_bf16_swiglu(fi_context* ctx, const void* d_a, int32_t a_dtype, int32_t lda, const uint16_t* d_bp_pair,

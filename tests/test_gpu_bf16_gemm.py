@@ -430,3 +430,27 @@ def test_bf16_swiglu_few_rows_route(gpu_ctx, m, k, n):
         narrow = torch.empty(m, n, device="cuda", dtype=torch.bfloat16)
         gpu_ctx.gemm_bf16_swiglu(a16[:, :k], pair, k, n, narrow, *b)
         assert torch.equal(narrow, outs[0].bfloat16())
+
+
+@pytest.mark.parametrize("n", [32768, 32784, 65536, 65552])
+@pytest.mark.parametrize("m,k", [(1, 72), (16, 2047), (16, 2048), (17, 2048), (17, 2049), (32, 40), (33, 72), (64, 40)])
+def test_bf16_wide_few_rows_route(gpu_ctx, m, k, n):
+    """Wide products of up to 64 rows (a head's logits) on both sides of each choice between the
+    two kernels, in one split and in the library's count, against f64 on the same bf16 operands
+    (1e-5 normwise: only f32 sums differ); f32 and bf16 rows agree bit for bit."""
+    import torch
+
+    print(f"bf16 wide few rows m={m} k={k} n={n}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m + k + n)
+    a16 = torch.full((m, (k + 7) // 8 * 8), float("nan"), device="cuda", dtype=torch.bfloat16)
+    a16[:, :k] = torch.randn(m, k, generator=g, device="cuda")
+    w = (torch.randn(k, n, generator=g, device="cuda") * 0.02).bfloat16()
+    want = a16[:, :k].double() @ w.double()
+    bp = gpu_ctx.weight_pack_bf16(w, k, n)
+    for splits in sorted({1, gpu_ctx.gemm_bf16_splits(m, k, n)}):
+        outs = []
+        for a in (a16, a16.float()):
+            outs.append(torch.full((splits, m, n), float("nan"), device="cuda"))
+            gpu_ctx.gemm_bf16(a[:, :k], bp, k, n, splits, outs[-1])
+        assert torch.equal(outs[0], outs[1])
+        assert ((outs[0].double().sum(dim=0) - want).norm() / want.norm()).item() <= 1e-5

@@ -428,12 +428,15 @@ __device__ __forceinline__ void split3(const f32x8& x, bf16x8& hi, bf16x8& mid, 
 constexpr int kTermA[6] = {2, 0, 1, 1, 0, 0};
 constexpr int kTermB[6] = {0, 2, 1, 0, 1, 0};
 
-// Three workgroups a CU (168 registers, 48 KiB of LDS each): counters of two showed the MFMAs busy
-// 34 % of the time, the split's VALU work 29 % and the waves waiting for the rest, so a third wave
-// a SIMD fills in (w1|w3 at 914 rows 134 -> 122 us, the 64-row greedy head 170 -> 156 us,
-// 200 rows 583 -> 538 us).  The K-tail form would spill there and keeps two.
+// 168 registers and 48 KiB of LDS, so three workgroups share a CU where the grid has them (w1|w3 at
+// 512 rows, 608 workgroups 72.9 -> 63.0 us, the 64-row greedy head, 1187, 171 -> 157, 200 rows 584 ->
+// 532).  The launch bound still asks for two waves a SIMD: asked for three the compiler reaches the
+// same register count, but grids without a third workgroup ran slower than with two (us: two
+// waves at 182 registers / three asked / two asked at 168; 256 x 688, K 256, 8 x 11 workgroups 11.8
+// / 13.8 / 11.9; w1|w3 at 128 rows, 152 workgroups 34.5 / 36.5 / 34.8).  The K-tail form takes 170
+// and keeps two.
 template <int MT, int PW, int EPI, bool KTAIL>
-__global__ __launch_bounds__(kThreads, KTAIL ? 2 : 3) void gemm_s3_kernel(PGemmArgs g) {
+__global__ __launch_bounds__(kThreads, 2) void gemm_s3_kernel(PGemmArgs g) {
   using BV = typename PVec<PW>::T;
   constexpr int KC = 2;                 // 32-k steps per staged A chunk
   constexpr int R = 2 * KC;             // B ring slots span two chunks: slot of step j of chunk c = (c % 2) KC + j

@@ -1013,15 +1013,32 @@ namespace {
 // launch of few workgroups is bound by one workgroup's serial chain, most of it arithmetic in
 // proportion to its heads, so it is cut by heads while the chip has room: each share reads the
 // same K/V (through one L2, see head_unit) and computes its heads exactly as the whole group's
-// workgroup would, so outputs do not depend on the cut.  In two while that leaves two workgroups
-// per CU, in four while it leaves one (us, 1 / 2 / 4 shares):
-//   7 heads, D 64, f32: 1 sequence of 700 tokens 12.9 / 9.6 / 8.3, 16 of 64-200 9.4 / 7.2 / 6.0,
-//     32 of 64-1000 (256 workgroups) 14.4 / 12.1 / 17.0;
-//   4 heads, D 128, f32: 8 of 200-400 (64 workgroups) 14.3 / 11.4 / 10.1, 16 (128) 14.7 / 11.8 / 13.2;
-//   4 heads, D 128, bf16: 1 of 1000 16.4 / 12.7 / 10.7, 8 of 200-2000 (256) 16.9 / 15.2.
-int head_split(int64_t whole, int group, int64_t cus) {
-  if (group >= 4 && 4 * whole <= cus) return 4;
-  return group >= 2 && 2 * whole <= 2 * cus ? 2 : 1;
+// workgroup would, so outputs do not depend on the cut.  The cut pays while the heads' arithmetic
+// outweighs reading K/V twice over, so the bound on `whole`, the launch's whole-group workgroups,
+// follows the heads a loaded byte serves, and long contexts (many full partitions) lower it where
+// those are few (us, 1 / 2 / 4 shares; w: whole on 256 CUs):
+//   7 heads, D 64, f32: 1 sequence of 700 tokens 12.9 / 9.6 / 8.3; w 256, 16 of 200-2000 13.4 / 11.6 /
+//     11.8, 4 of 3000-8000 16.7 / 15.3 / 16.0; w 512, 32 of 200-2000 16.6 / 18.1 / 19.2;
+//   4 heads, D 128, f32: w 64, 8 of 200-400 14.3 / 11.4 / 10.1; w 192, 6 of 200-2000 17.9 / 17.4 / 18.8;
+//     w 256, 8 of 200-2000 18.8 / 19.9 / 30.2, 2 of 3000-8000 21.2 / 26.0 / 52.7, but 32 of 60-250 (one
+//     partition) 14.2 / 13.6 / 19.8;
+//   4 heads, D 128, bf16: w 256, 8 of 200-2000 16.9 / 15.7 / 18.4; w 512, 16 22.6 / 25.2 / 35.3;
+//   4 heads, D 32, f32, 3000-8000: w 64 9.2 / 9.0 / 10.1, w 128 9.6 / 9.8 / 11.9, w 256 10.6 / 12.0 / 14.3;
+//   2 heads, D 128, f32: w 128, 8 of 300-700 13.5 / 12.7, 1 of 3000-8000 16.1 / 17.4; w 192, 6 of 200-2000
+//     15.0 / 16.4.
+int head_split(int64_t whole, int group, int parts, bool bf16, int64_t cus) {
+  const bool many = parts > 16 && group <= 4;
+  if (group >= 4 && 4 * whole <= cus && !many) return 4;
+  if (group < 2) return 1;
+  int64_t limit = cus;  // of the launches cut in two
+  if (many) {
+    limit = group == 2 ? 0 : cus / 4;
+  } else if (group == 2) {
+    limit = parts > 8 ? 0 : cus / 2;
+  } else if (group <= 4 && !bf16 && parts > 1) {
+    limit = 3 * cus / 4;
+  }
+  return whole <= limit ? 2 : 1;
 }
 
 // Shared by both decode entry points: validation, launch shape and launches.  With
@@ -1137,7 +1154,7 @@ int32_t decode_paged(fi_context* ctx, const float* d_q, const void* d_k_cache, c
   }
   const int64_t cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
   const int64_t whole = static_cast<int64_t>(num_seqs) * num_kv_heads * parts;  // workgroups with whole groups
-  const int shares = head_split(whole, args.group, cus);
+  const int shares = head_split(whole, args.group, parts, kv_dtype == FI_DTYPE_BF16, cus);
   args.heads_per = (args.group + shares - 1) / shares;
   const dim3 grid(static_cast<unsigned>(whole), static_cast<unsigned>(shares));
   // Small launches (at most six workgroups a CU, e.g. a decode tick of a small model) merge

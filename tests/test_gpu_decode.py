@@ -526,3 +526,38 @@ def test_decode_head_shares_do_not_change_outputs(gpu_ctx, kv_dtype, hq, hkv, d)
         for a, b in zip(got[2:], whole[2:]):
             assert torch.equal(a[used // bs, :, used % bs], b[used // bs, :, used % bs])
     gpu_ctx.check_faults()
+
+
+@pytest.mark.parametrize("kv_dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("hq,hkv,d", [(4, 2, 32), (8, 2, 32), (14, 2, 64)])
+def test_decode_head_shares_of_long_contexts(gpu_ctx, kv_dtype, hq, hkv, d):
+    """More than 16 partitions a sequence, where groups of up to four heads are cut less: one, three
+    and seven sequences give the bits they give in a batch that is not cut."""
+    import torch
+
+    from ferrisinfer_amd import DTYPE_BF16, DTYPE_F32
+
+    print(f"head shares long {hq}/{hkv} d={d} {kv_dtype}", flush=True)
+    bs, dt = 16, DTYPE_F32 if kv_dtype == "f32" else DTYPE_BF16
+    lens = np.array([4400, 300, 17, 4353, 1, 2048, 4096, 700, 4399], np.int32)
+    nblk = (lens + bs - 1) // bs
+    at = np.concatenate([[0], np.cumsum(nblk)])
+    order = np.random.default_rng(hq + d).permutation(int(at[-1])).astype(np.int32)
+    tables = np.zeros((len(lens), int(nblk.max())), np.int32)
+    for i, k in enumerate(nblk):
+        tables[i, :k] = order[at[i]:at[i + 1]]
+    g = torch.Generator(device="cuda").manual_seed(hq * d)
+    k, v = (torch.randn(int(at[-1]), hkv, bs, d, generator=g, device="cuda").to(
+        torch.float32 if kv_dtype == "f32" else torch.bfloat16) for _ in range(2))
+    q = torch.randn(len(lens), hq, d, generator=g, device="cuda")
+
+    def run(n):
+        out = torch.full((n, hq, d), float("nan"), device="cuda")
+        gpu_ctx.attn_decode_paged(q[:n].contiguous(), k, v, dt, _dev(tables[:n].copy(), torch), _dev(lens[:n].copy(), torch),
+                                  int(lens.max()), hkv, bs, int(at[-1]), d ** -0.5, out)
+        return out
+
+    whole = run(len(lens))
+    for n in (1, 3, 7):
+        assert torch.equal(run(n), whole[:n]), n
+    gpu_ctx.check_faults()

@@ -13,9 +13,10 @@
 // which is the B operand of one 16x16x32 MFMA per (slab, step) for lane `lane`: every wave
 // load is 16 contiguous bytes per lane and one group's K step is 16 KiB contiguous.
 //
-// Kernel (above 64 rows, and the greedy head): a workgroup of 4 waves computes a (16 MT) x (64 NT)
-// tile over one split's K range (MT = 8, 6 or 4 row tiles above 64 rows, chosen per shape so the busiest CU gets the least
-// work).  The activation block (16 MT rows x 32 k, or 64 k for bf16 activations) is staged per
+// Tile kernel (above 64 rows, the greedy head, and the shapes of fewer rows that rows_product and
+// rows_swiglu leave to it): a workgroup of 4 waves computes a (16 MT) x (64 NT) tile over one
+// split's K range (MT = 8, 6 or 4 row tiles above 64 rows, chosen per shape so the busiest CU gets
+// the least work).  The activation block (16 MT rows x 32 k, or 64 k for bf16 activations) is staged per
 // step through double-buffered LDS: f32 activations are rounded to bf16 (nearest even) on the
 // way in, bf16 activations (rounded the same way by their producer) are copied, so both give
 // the same products; bf16 halves the bytes the vector memory path carries per step, which at
@@ -355,7 +356,8 @@ template <int MT, int NS, int SW, int KW, int DEPTH, int EPI, bool KTAIL, bool A
 __global__ __launch_bounds__(64 * SW * KW, 2) void gemm_bf16_rows_kernel(BGemmArgs g) {
   constexpr int AV = A16 ? 1 : 2;              // 16-byte loads of an activation fragment and lane
   constexpr int FRAGS = DEPTH * MT;            // 1 KiB bf16 fragments of a part's stage
-  constexpr int A_PER = (FRAGS + SW - 1) / SW; // per wave
+  constexpr int A_PER = FRAGS / SW;            // per wave
+  static_assert(FRAGS % SW == 0 && KW > 1, "whole fragments a wave, parts that meet in LDS");
   constexpr int A_BYTES = 2 * KW * FRAGS * 1024, P_BYTES = KW * SW * MT * NS * 1024;
   __shared__ __align__(16) unsigned char s_mem[A_BYTES > P_BYTES ? A_BYTES : P_BYTES];
   uint4* const s_a = reinterpret_cast<uint4*>(s_mem);  // [2][KW][DEPTH][MT][64]
@@ -387,7 +389,7 @@ __global__ __launch_bounds__(64 * SW * KW, 2) void gemm_bf16_rows_kernel(BGemmAr
   auto load_a = [&](int stage) {
 #pragma unroll
     for (int r = 0; r < A_PER; ++r) {
-      const int f = min(sw + r * SW, FRAGS - 1);
+      const int f = sw + r * SW;
       const int kk = step_at(stage * DEPTH + f / MT) * kStepK + 8 * lk;
       const int row = min(16 * (f % MT) + li, g.m - 1);
       if constexpr (KTAIL) ak[r] = kk;
@@ -405,7 +407,6 @@ __global__ __launch_bounds__(64 * SW * KW, 2) void gemm_bf16_rows_kernel(BGemmAr
   auto store_a = [&](int buf) {
 #pragma unroll
     for (int r = 0; r < A_PER; ++r) {
-      if (FRAGS % SW != 0 && sw + r * SW >= FRAGS) continue;
       uint4 x = areg[r][0];
       if constexpr (!A16) {
         const float4 lo = __builtin_bit_cast(float4, areg[r][0]), hi = __builtin_bit_cast(float4, areg[r][1]);
@@ -467,30 +468,25 @@ __global__ __launch_bounds__(64 * SW * KW, 2) void gemm_bf16_rows_kernel(BGemmAr
   };
   for (int st = 0; st + 1 < nst; ++st) stage(st, std::true_type{});
   stage(nst - 1, std::false_type{});
-  if constexpr (KW == 1) {
-    store_tile<MT, NS, EPI>(g, acc, 0, slab0, z, lane);
-    return;
-  } else {
-    v4f* const s_part = reinterpret_cast<v4f*>(s_mem);  // [KW][SW][MT * NS][64]
+  v4f* const s_part = reinterpret_cast<v4f*>(s_mem);  // [KW][SW][MT * NS][64]
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
+  for (int t = 0; t < MT; ++t)
 #pragma unroll
-      for (int s = 0; s < NS; ++s) s_part[((kw * SW + sw) * MT * NS + t * NS + s) * 64 + lane] = acc[t][s];
-    __syncthreads();
-    // wave (sw, kw) adds and stores row tiles kw, kw + KW, ... of its slabs
+    for (int s = 0; s < NS; ++s) s_part[((kw * SW + sw) * MT * NS + t * NS + s) * 64 + lane] = acc[t][s];
+  __syncthreads();
+  // wave (sw, kw) adds and stores row tiles kw, kw + KW, ... of its slabs
 #pragma unroll
-    for (int t0 = 0; t0 < MT; t0 += KW) {
-      const int t = t0 + kw;
-      if (t >= MT) return;
-      v4f sum[1][NS];
+  for (int t0 = 0; t0 < MT; t0 += KW) {
+    const int t = t0 + kw;
+    if (t >= MT) return;
+    v4f sum[1][NS];
 #pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        sum[0][s] = s_part[(sw * MT * NS + t * NS + s) * 64 + lane];
+    for (int s = 0; s < NS; ++s) {
+      sum[0][s] = s_part[(sw * MT * NS + t * NS + s) * 64 + lane];
 #pragma unroll
-        for (int src = 1; src < KW; ++src) sum[0][s] += s_part[((src * SW + sw) * MT * NS + t * NS + s) * 64 + lane];
-      }
-      store_tile<1, NS, EPI>(g, sum, 16 * t, slab0, z, lane);
+      for (int src = 1; src < KW; ++src) sum[0][s] += s_part[((src * SW + sw) * MT * NS + t * NS + s) * 64 + lane];
     }
+    store_tile<1, NS, EPI>(g, sum, 16 * t, slab0, z, lane);
   }
 }
 

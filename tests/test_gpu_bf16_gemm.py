@@ -316,7 +316,8 @@ def test_convert_f32_to_bf16(orc, gpu_ctx, n, offset):
 
 
 @pytest.mark.parametrize("m", [1, 16, 17, 32, 33, 64, 65])
-@pytest.mark.parametrize("k,n", [(24, 4090), (1000, 4112), (4864, 896), (520, 8200)])
+@pytest.mark.parametrize("k,n", [(24, 4090), (1000, 4112), (4864, 896), (520, 8200), (1001, 4112), (525, 896),
+                                 (31, 8200)])
 def test_bf16_few_rows_edges(gpu_ctx, m, k, n):
     """Both sides of every row-tile and slab-count choice up to 64 rows (and the first row count
     past it), K shorter than one step, with a tail, an uneven last part and several stages:

@@ -468,12 +468,20 @@ def test_prefill_order_without_plan(gpu_ctx, hq, hkv, d, kv):
         cu = np.concatenate([[0], np.cumsum([n for _, n in seqs])]).astype(np.int32)
         q = torch.randn(int(cu[-1]), hq, d, generator=g, device="cuda")
         out = torch.full_like(q, float("nan"))
-        args = (tables, torch.from_numpy(cu).cuda(), torch.tensor(lens, dtype=torch.int32, device="cuda"),
-                max(n for _, n in seqs) + slack, hkv, bs, at, d ** -0.5, out)
-        if kv == "bf16-mfma":
-            gpu_ctx.attn_prefill_paged_bf16(q, k, v, *args)
-        else:
-            gpu_ctx.attn_prefill_paged(q, k, v, DTYPE_F32 if kv == "f32" else DTYPE_BF16, *args)
+        ends, lens_dev = torch.from_numpy(cu).cuda(), torch.tensor(lens, dtype=torch.int32, device="cuda")
+
+        def run(rows, table, ends, lens, longest, dst):
+            args = (table, ends, lens, longest, hkv, bs, at, d ** -0.5, dst)
+            if kv == "bf16-mfma":
+                gpu_ctx.attn_prefill_paged_bf16(rows, k, v, *args)
+            else:
+                gpu_ctx.attn_prefill_paged(rows, k, v, DTYPE_F32 if kv == "f32" else DTYPE_BF16, *args)
+
+        run(q, tables, ends, lens_dev, max(n for _, n in seqs) + slack, out)
+        alone = torch.full_like(q, float("nan"))
+        for i, (_, n) in enumerate(seqs):
+            run(q[cu[i]:cu[i + 1]], tables[i:i + 1].contiguous(), ends[i:i + 2] - ends[i], lens_dev[i:i + 1], n,
+                alone[cu[i]:cu[i + 1]])
         want = torch.empty_like(q, dtype=torch.float64)
         for i, (p, n) in enumerate(seqs):
             ids = tables[i, :nblk[i]].long()
@@ -483,6 +491,7 @@ def test_prefill_order_without_plan(gpu_ctx, hq, hkv, d, kv):
                 j = h // (hq // hkv)
                 s = (q[cu[i]:cu[i + 1], h].double() @ keys[:, j].t()) * d ** -0.5
                 want[cu[i]:cu[i + 1], h] = torch.softmax(s.masked_fill(mask, float("-inf")), dim=1) @ vals[:, j]
-        err = ((out.double() - want).norm() / want.norm()).item()
-        assert err <= (1e-2 if kv == "bf16-mfma" else 1e-5), (seqs, err)
+        for got in (out, alone):
+            err = ((got.double() - want).norm() / want.norm()).item()
+            assert err <= (1e-2 if kv == "bf16-mfma" else 1e-5), (seqs, err)
     gpu_ctx.check_faults()

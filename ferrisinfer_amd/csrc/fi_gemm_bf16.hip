@@ -347,7 +347,10 @@ __global__ __launch_bounds__(kThreads, kOccupancy) void gemm_bf16_kernel(BGemmAr
 // registers at the start of the stage before (ahead of that stage's weight loads, which return
 // after them and so stay in flight at its end), then put in LDS in fragment order, where the SW
 // waves of the part share them.  The KW partial sums meet in LDS and are added in part order, so
-// a consumer reads a few partials instead of up to 32, and SwiGLU needs none.
+// a consumer reads a few partials instead of up to 32, and SwiGLU needs none.  A stage is summed by
+// itself before it joins its part: a running sum over all of a part's K is longer than a split's
+// of the tile kernel and less exact (16 rows of w1|w3, f32 SwiGLU against 64 bits, normwise: 4.1e-7;
+// the tile kernel 2.2e-7; by stages 1.65e-7, and no slower: 42 us).
 // Llama-3-8B's MLP, weights from HBM, against the kernel above: 16 rows, w1|w3 51 + 4.8 (its split
 // sum) -> 42.5 us (5.5 TB/s), w2 24 -> 22 us (5.3 TB/s); 64 rows, 69.7 + 9.4 -> 51 us and
 // 32.5 -> 29.3 us.  What is left over a plain stream grows with the rows: each workgroup reads
@@ -428,11 +431,11 @@ __global__ __launch_bounds__(64 * SW * KW, 2) void gemm_bf16_rows_kernel(BGemmAr
       s_a[((buf * KW + kw) * FRAGS + sw + r * SW) * 64 + lane] = x;
     }
   };
-  v4f acc[MT][NS];
+  v4f total[MT][NS];
 #pragma unroll
   for (int t = 0; t < MT; ++t)
 #pragma unroll
-    for (int s = 0; s < NS; ++s) acc[t][s] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < NS; ++s) total[t][s] = v4f{0.f, 0.f, 0.f, 0.f};
 
   load_a(0);
   sched_fence();
@@ -446,6 +449,11 @@ __global__ __launch_bounds__(64 * SW * KW, 2) void gemm_bf16_rows_kernel(BGemmAr
       load_a(st + 1);
       sched_fence();
     }
+    v4f acc[MT][NS];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int s = 0; s < NS; ++s) acc[t][s] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) {
       const int step = st * DEPTH + d;
@@ -463,6 +471,10 @@ __global__ __launch_bounds__(64 * SW * KW, 2) void gemm_bf16_rows_kernel(BGemmAr
       if constexpr (decltype(more)::value) issue(step + DEPTH, ring[d]);
       sched_fence();
     }
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int s = 0; s < NS; ++s) total[t][s] += acc[t][s];
     if constexpr (decltype(more)::value) store_a((st & 1) ^ 1);
     __syncthreads();
   };
@@ -472,7 +484,7 @@ __global__ __launch_bounds__(64 * SW * KW, 2) void gemm_bf16_rows_kernel(BGemmAr
 #pragma unroll
   for (int t = 0; t < MT; ++t)
 #pragma unroll
-    for (int s = 0; s < NS; ++s) s_part[((kw * SW + sw) * MT * NS + t * NS + s) * 64 + lane] = acc[t][s];
+    for (int s = 0; s < NS; ++s) s_part[((kw * SW + sw) * MT * NS + t * NS + s) * 64 + lane] = total[t][s];
   __syncthreads();
   // wave (sw, kw) adds and stores row tiles kw, kw + KW, ... of its slabs
 #pragma unroll
@@ -864,7 +876,7 @@ int32_t fi_gemm_bf16_splits(fi_context* ctx, int32_t m, int32_t k, int32_t n, in
   FI_REQUIRE(m >= 0 && k > 0 && n > 0, FI_ERR_INVALID_SHAPE, "fi_gemm_bf16_splits: bad shape");
   FI_REQUIRE(splits != nullptr, FI_ERR_INVALID_CONFIG, "fi_gemm_bf16_splits: null output");
   const int slabs = data_slabs(n, false);
-  *splits = m <= kRowsMax ? rows_splits(ctx, q_steps(k), slabs) : tile_splits(ctx, m, k, slabs);
+  *splits = rows_product(ctx, m, k, slabs) ? rows_splits(ctx, q_steps(k), slabs) : tile_splits(ctx, m, k, slabs);
   return FI_OK;
 }
 

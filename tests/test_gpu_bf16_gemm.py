@@ -455,3 +455,35 @@ def test_bf16_wide_few_rows_route(gpu_ctx, m, k, n):
             gpu_ctx.gemm_bf16(a[:, :k], bp, k, n, splits, outs[-1])
         assert torch.equal(outs[0], outs[1])
         assert ((outs[0].double().sum(dim=0) - want).norm() / want.norm()).item() <= 1e-5
+
+
+@pytest.mark.parametrize("k,n", [(256, 688), (896, 4864), (4096, 4096), (4096, 14336), (14336, 4096)])
+def test_bf16_few_rows_are_as_exact_as_many(gpu_ctx, k, n):
+    """Products are exact in f32, so a kernel's distance from 64 bits is that of its f32 sums: with
+    up to 64 rows no further off than the same rows in a call of 65, which takes row tiles.  5 %
+    more is left for the spread of the mean over at least 16 x 688 values (about 1 %)."""
+    import torch
+
+    print(f"bf16 few rows exactness k={k} n={n}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(k + n)
+    a = torch.randn(65, k, generator=g, device="cuda").bfloat16()
+    w1, w3 = ((torch.randn(k, n, generator=g, device="cuda") * 0.02).bfloat16() for _ in range(2))
+    up, gate = a.double() @ w1.double(), a.double() @ w3.double()
+    want = up, up * torch.nn.functional.silu(gate)
+    bp, pair = gpu_ctx.weight_pack_bf16(w1, k, n), gpu_ctx.weight_pack_bf16_pair(w1, w3, k, n)
+
+    def run(m):
+        splits = gpu_ctx.gemm_bf16_splits(m, k, n)
+        parts, act = torch.empty(splits, m, n, device="cuda"), torch.empty(m, n, device="cuda")
+        gpu_ctx.gemm_bf16(a[:m], bp, k, n, splits, parts)
+        gpu_ctx.gemm_bf16_swiglu(a[:m], pair, k, n, act)
+        total = parts[0].clone()
+        for p in parts[1:]:  # f32, in split order, as the consumers add them
+            total += p
+        return total, act
+
+    many = run(65)
+    for m in (16, 32, 64):
+        for few, ref, exact in zip(run(m), many, want):
+            off = [(x[:m].double() - exact[:m]).norm().item() for x in (few, ref)]
+            assert off[0] <= 1.05 * off[1], (m, off)

@@ -107,7 +107,7 @@ __device__ __forceinline__ void load_step(const float* row, int vocab, int s, in
 // to its use.  Those steps load step nsteps - 1 again, which the range has just read, instead
 // of the logits past the range (another segment's, which would be read from memory twice).
 // prime_steps issues no load for a slot past the range: a short row's repeats would queue ahead
-// of its own (4096 logits, top-k 20: 9.8 -> 9.0 us for one row; 1000, top-k 2: 8.7 -> 8.2).
+// of its own (top-k 20, one row of 4096: 9.8 -> 9.2 us, 257 rows of 1000 18.2 -> 17.9).
 // Four buffers: three primed ones leave the bound below a quarter fewer logits, five spill
 // (64 rows of 151936, top-k 20: 21.2 us with four, 21.9 with five).
 constexpr int kRing = 4;
@@ -1049,10 +1049,11 @@ __device__ __forceinline__ void write_token(SampleShared& sh, const float* row, 
 
 // ---- launch 1: one workgroup per (row segment, row) ----
 // Segment j covers wave steps [j * seg_steps, (j + 1) * seg_steps).  Greedy rows leave their
-// segment's partial; sampled rows with k < vocab and k <= 1024 leave every logit of the segment
-// at or above the segment's k+1-th largest (a superset of the row's top k+1 that lies in the
-// segment) in the workspace, unordered; a flag (NaN, overflow, more than one region of
-// candidates) sends the row to the full replay in the finish.
+// segment's partial; sampled rows with k < vocab and k <= 1024 leave candidates in the workspace,
+// unordered: a superset of the segment's k+1 largest logits.  It is all that was buffered where
+// that is at most k + 1 or few enough for the finish to take as it is (`direct` below), else every
+// logit at or above the segment's k+1-th largest.  A flag (NaN, overflow, more than one region
+// of candidates) sends the row to the full replay in the finish.
 template <int VEC>
 __global__ __launch_bounds__(kThreads) void sample_scan_kernel(const float* __restrict__ logits, int ld, int vocab,
                                                                int segs, int seg_steps,
@@ -2070,8 +2071,11 @@ int32_t fi_sample_tokens(fi_context* ctx, const float* d_logits, int32_t ld, int
   FI_REQUIRE(d_logits && d_temperature && d_top_k && d_top_p && d_rng_state && d_token && d_prob,
              FI_ERR_INVALID_CONFIG, "fi_sample_tokens: null pointer");
   FI_REQUIRE(rows <= 65535, FI_ERR_INVALID_SHAPE, "fi_sample_tokens: at most 65535 rows per call");
-  // rows split only as far as it takes to give every CU a workgroup (one fits a CU): a short
-  // segment buffers nearly all of its logits, so more segments cost more than they spread.
+  // rows split only as far as it takes to give every CU a workgroup (one fits a CU): a second round
+  // of workgroups costs more than shorter segments save (64 rows of 151936, top-k 20, in 1 / 2 / 4 /
+  // 8 segments 27.6 / 24.1 / 20.6 / 26.8 us; 16 rows 25.4 / 21.6 / 17.6 / 16.9).  Rows of up to 32000
+  // logits would now run faster in one segment, without the finish's launch (one row of 8192, top-k
+  // 20: 11.1 in two, 8.6 in one; 64 rows of 32000 13.5 in four, 12.6 in one).
   // Segments hold at least four wave steps (4096 logits, more than k + 1 for any k the device
   // takes) and at most one per wave buffer of the finish.
   const int nsteps = (vocab + kStep - 1) / kStep;

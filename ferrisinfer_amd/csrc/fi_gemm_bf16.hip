@@ -527,7 +527,9 @@ void launch_rows_as(fi_context* ctx, const BGemmArgs& g) {
 
 // Slabs a workgroup of the split-K products owns: eight (4 x 2 waves of two slabs), or four where
 // that would leave fewer than 32 workgroups a split (56 slabs, K 4864, 64 rows: 6.1 us against
-// 8.9 us of the kernel above).
+// 8.9 us of the kernel above).  Four against eight, K 4096 with the norm behind it, us: 64 slabs, 64
+// rows 11.6 / 13.0; 128 slabs 12.8 / 14.2; 384 slabs 38.3 / 24.1, 16 rows 22.5 / 17.9.  Between, either
+// wins by up to a tenth (192 slabs, 64 rows 18.3 / 16.6; 256, 16 rows 14.1 / 13.5; 320 16.7 / 18.2).
 int rows_slabs(int slabs) { return slabs >= 256 ? 8 : 4; }
 
 template <int MT, int EPI, bool A16>

@@ -1222,8 +1222,8 @@ int split_count(fi_context* ctx, int m, int k, int slabs, int pw) {
 
 // Pack width 32: 32-row tiles (one for M <= 32, else two per workgroup), and two slabs per
 // workgroup once that still gives half the CUs a workgroup (prefill M); at decode M one slab,
-// with K split until the grid is one workgroup per CU, every split at least 8 steps.  Timed on
-// the box at the C4 shapes against the f32-MFMA kernels: M = 64 q|k|v 8.3 -> 6.7 us (7
+// with K split until the grid is one workgroup per CU, every split at least 8 steps.  Timed
+// at the C4 shapes against the f32-MFMA kernels: M = 64 q|k|v 8.3 -> 6.7 us (7
 // splits), wo 8.3 -> 6.5 us (7), w2 12.2 -> 11.1 us (9); M = 1024 (one split, two slabs) q|k|v
 // 41.8 -> 31.3 us, wo 24.8 -> 19.9 us, w2 83.9 -> 74.0 us.
 struct W32Plan {
